@@ -51,14 +51,59 @@ constexpr int kStreamKSpinLimit = 1 << 22;
 // Variants: whole 64x64 tiles per workgroup (BK 64 or 32), or stream-K
 // (BK 64); kAuto takes CJ_HIP_GEMM_F32=dp|sk|bk32, else the heuristic of
 // gemmF32Choose.
-enum class GemmF32Variant { kAuto = 0, kDataParallel = 1, kStreamK = 2, kDataParallelBK32 = 3 };
+enum class GemmF32Variant {
+  kAuto = 0, kDataParallel = 1, kStreamK = 2, kDataParallelBK32 = 3, kSplit64 = 4, kSplit80 = 5, kSplit128 = 6
+};
 GemmF32Variant gemmF32Choose(int M, int N, int max_groups);
 hipError_t gemmF32Padded(const float* A, const float* B, float* C, int M, int N, int K, int lda, int ldb, int ldc,
                          const StreamKSync& sync, int max_groups, GemmF32Variant variant, hipStream_t stream);
+// Whether both padded operands of a split GEMM hold only values that three
+// bf16 parts represent exactly, as found while they were copied: an operand's
+// word equals its epoch when padCopyF32 met another value (it is never
+// cleared; every copy has a new epoch).
+struct SplitGuardF32 {
+  const int* word_a;
+  const int* word_b;
+  int epoch_a;
+  int epoch_b;
+  __device__ bool unsafe() const { return *word_a == epoch_a || *word_b == epoch_b; }
+};
+// An operand of the split GEMM: the padded fp32 matrix (A [16 bands, K] or B
+// [K, 16 bands], row stride ld) and its three bf16 planes, 16 * bands * K
+// values each (splitPlanesF32 writes them).
+struct SplitOperandF32 {
+  const float* src;
+  int ld;
+  int bands;
+  uint16_t* planes;
+};
+// Workspace of a GEMM whose tiles are shared by several workgroups along k:
+// partial tiles and one counter per tile (zero at allocation, left at zero by
+// every launch).  Launches that share it must not overlap.
+struct SplitKWork {
+  float* part;
+  int* counters;
+};
+// Writes the planes of the operands whose src is not null; K a multiple of 64.
+hipError_t splitPlanesF32(const SplitOperandF32& a, const SplitOperandF32& b, int K, hipStream_t stream);
+// C [M, N] (ldc) = A . B from the planes (gemm_f32.hip): variants kSplit64 and
+// kSplit80 (64 or 80 rows by 64 columns a workgroup) and kSplit128 (128 x
+// 128); `splits` workgroups share a tile's k range, with `work` holding
+// gemmF32SplitPartFloats * splits floats and one counter per tile.
+hipError_t gemmF32Split(const SplitOperandF32& A, const SplitOperandF32& B, float* C, int M, int N, int K, int ldc,
+                        const SplitGuardF32& guard, const SplitKWork& work, GemmF32Variant variant, int splits,
+                        hipStream_t stream);
+int gemmF32SplitTiles(GemmF32Variant variant, int M, int N);
+size_t gemmF32SplitPartFloats(GemmF32Variant variant);
+// The workgroups per tile and the variant for a problem on `cus` CUs.
+int gemmF32SplitCount(GemmF32Variant variant, int M, int N, int K, int cus);
+GemmF32Variant gemmF32SplitChoose(int M, int N, int K, int cus);
 // dst[r][c] = src[r][c] (row stride ld_src) for r < rows, c < cols; 0 up to
-// rows_pad x cols_pad (dst row stride cols_pad).
+// rows_pad x cols_pad (dst row stride cols_pad).  With `guard`, *guard and
+// *guard_host (device-mapped host memory) become `epoch` if a value is an
+// infinity, a NaN or not 0 and outside [2^-100, 2^50].
 hipError_t padCopyF32(const float* src, float* dst, int rows, int cols, size_t ld_src, int rows_pad, int cols_pad,
-                      hipStream_t stream);
+                      hipStream_t stream, int* guard = nullptr, int* guard_host = nullptr, int epoch = 0);
 // out2d = cols[M,K] . Wt^T where Wt is [N,K] (conv weights as stored, OIHW);
 // epilogue adds bias, applies ReLU and scatters to NCHW out[img, n, pix]
 // (m = img*ohw + pix).

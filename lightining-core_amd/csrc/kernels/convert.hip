@@ -79,12 +79,14 @@ __global__ __launch_bounds__(256) void convert_pad_kernel(const float* __restric
 
 __global__ __launch_bounds__(256) void pad_copy_f32_kernel(const float* __restrict__ src, float* __restrict__ dst,
                                                            int rows, int cols, size_t ld_src, int rows_pad,
-                                                           int cols_pad) {
+                                                           int cols_pad, int* __restrict__ guard,
+                                                           int* __restrict__ guard_host, int epoch) {
   // 4 output elements per thread along the padded row; cols_pad % 4 == 0.
   const int c4 = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (c4 >= cols_pad) {
     return;
   }
+  bool odd = false;  // a value that three bf16 parts may not hold
   for (int r = blockIdx.y; r < rows_pad; r += gridDim.y) {
     float4 v;
     float* pv = reinterpret_cast<float*>(&v);
@@ -92,8 +94,14 @@ __global__ __launch_bounds__(256) void pad_copy_f32_kernel(const float* __restri
     for (int j = 0; j < 4; ++j) {
       const int c = c4 + j;
       pv[j] = (r < rows && c < cols) ? src[static_cast<size_t>(r) * ld_src + c] : 0.0f;
+      const uint32_t mag = __builtin_bit_cast(uint32_t, pv[j]) & 0x7fffffffu;
+      odd |= mag != 0 && (mag < 0x0d800000u || mag > 0x58800000u);  // 2^-100, 2^50
     }
     *reinterpret_cast<float4*>(dst + static_cast<size_t>(r) * cols_pad + c4) = v;
+  }
+  if (guard != nullptr && odd) {
+    *guard = epoch;  // every writer stores the same value
+    __hip_atomic_store(guard_host, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -272,13 +280,13 @@ hipError_t vitPatchify(const float* x, uint16_t* xp, int B, int C, int H, int W,
 }
 
 hipError_t padCopyF32(const float* src, float* dst, int rows, int cols, size_t ld_src, int rows_pad, int cols_pad,
-                      hipStream_t stream) {
+                      hipStream_t stream, int* guard, int* guard_host, int epoch) {
   if (rows_pad <= 0 || cols_pad <= 0 || cols_pad % 4 != 0 || rows > rows_pad || cols > cols_pad) {
     return hipErrorInvalidValue;
   }
   const dim3 grid((cols_pad + 1023) / 1024, rows_pad < 65535 ? rows_pad : 65535);
   hipLaunchKernelGGL(pad_copy_f32_kernel, grid, dim3(256), 0, stream, src, dst, rows, cols, ld_src, rows_pad,
-                     cols_pad);
+                     cols_pad, guard, guard_host, epoch);
   return hipGetLastError();
 }
 

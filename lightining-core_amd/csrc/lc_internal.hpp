@@ -12,6 +12,7 @@
 #include <cstdint>
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "lightning_core_hip.h"
 
@@ -120,6 +121,7 @@ class PinnedBuffer {
   std::size_t bytes_ = 0;
 };
 
+constexpr int kGuardSlots = 1024;
 struct HipContext {
   std::recursive_mutex mu;
   int device = 0;
@@ -138,6 +140,17 @@ struct HipContext {
   // Split-K workspace of the skinny 16-bit GEMM (partials + per-column-tile
   // counters, zero at allocation and after every launch); `stream` only.
   DeviceBuffer skinny_part, skinny_counters;
+  // The same for GEMMs that split k over workgroups (kern::SplitKWork).
+  DeviceBuffer splitk_part, splitk_counters;
+  // Guard words of the fp32 split GEMM's operands (kern::SplitGuardF32), a
+  // pair per MatMulResident that holds a slot: the kernels' words and the
+  // host's copies.  kGuardSlots pairs, allocated once; a resident that gets no
+  // slot runs the fp32 kernels.  Epochs are unique over all slots, so a slot
+  // needs no clearing between owners.
+  DeviceBuffer guard_words;
+  PinnedBuffer guard_host;
+  std::vector<int> guard_free;
+  int guard_epoch = 0;
   // Enqueue-only launches since the stream was last synchronised, per op
   // family (noteEnqueued; syncStream resets both).
   std::size_t matmul_inflight = 0;

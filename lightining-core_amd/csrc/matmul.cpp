@@ -14,6 +14,7 @@
 // 16-bit compute rounds the fp32 host data once at upload (RNE) and lays B out
 // K-contiguous (transposed), the layout the MFMA GEMM reads.
 #include <algorithm>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -28,6 +29,59 @@ namespace lchip {
 
 namespace {
 
+// fp32 operands are scanned while they are padded (`which` 0: A, 1: B): the
+// words of the split GEMM's guard, and the epoch of this copy (every copy has
+// a new one, so the words are never cleared).
+struct GuardArgs {
+  int* word;  // null: not guarded
+  int* host;  // device alias
+  int epoch;
+};
+GuardArgs beginGuarded(HipContext* ctx, MatMulResident& r, int which) {
+  int& epoch = which == 0 ? r.epoch_a : r.epoch_b;
+  epoch = 0;
+  (which == 0 ? r.has_planes_a : r.has_planes_b) = false;
+  if (ctx->guard_host.get() == nullptr) {
+    const std::size_t bytes = 2 * kGuardSlots * sizeof(int);
+    if (ctx->guard_words.ensure(bytes, true) != Status::kSuccess ||
+        ctx->guard_host.ensure(bytes) != Status::kSuccess) {
+      return GuardArgs{nullptr, nullptr, 0};
+    }
+    std::memset(ctx->guard_host.get(), 0, bytes);
+    for (int i = kGuardSlots - 1; i >= 0; --i) {
+      ctx->guard_free.push_back(i);
+    }
+  }
+  if (r.guard_slot < 0 && !ctx->guard_free.empty()) {
+    r.guard_slot = ctx->guard_free.back();
+    ctx->guard_free.pop_back();
+  }
+  if (r.guard_slot < 0 || ctx->guard_epoch == INT_MAX) {
+    return GuardArgs{nullptr, nullptr, 0};
+  }
+  epoch = ++ctx->guard_epoch;
+  const int at = 2 * r.guard_slot + which;
+  return GuardArgs{ctx->guard_words.as<int>() + at, static_cast<int*>(ctx->guard_host.device()) + at, epoch};
+}
+
+void releaseGuard(HipContext* ctx, MatMulResident& r) {
+  if (r.guard_slot >= 0) {
+    ctx->guard_free.push_back(r.guard_slot);
+    r.guard_slot = -1;
+  }
+}
+
+// Whether an operand was not guarded, or the host has already seen that it is
+// unfit for the split (its upload has finished; until then the kernel's own
+// check decides).
+bool knownUnsafe(const HipContext* ctx, const MatMulResident& r) {
+  if (r.epoch_a == 0 || r.epoch_b == 0) {
+    return true;
+  }
+  const volatile int* w = static_cast<const volatile int*>(ctx->guard_host.get()) + 2 * r.guard_slot;
+  return w[0] == r.epoch_a || w[1] == r.epoch_b;
+}
+
 Status uploadA(HipContext* ctx, MatMulResident& r, const float* a) {
   if (!isHalf(r.dtype)) {
     // fp32: A [roundup(M, 64), roundup(K, 64)], zero pads
@@ -36,9 +90,10 @@ Status uploadA(HipContext* ctx, MatMulResident& r, const float* a) {
     LC_TRY(r.stage.ensure(r.m * r.k * sizeof(float)));
     LC_TRY(r.a.ensure(mp * kp * sizeof(float)));
     LC_TRY(upload(ctx, r.stage.get(), a, r.m * r.k * sizeof(float)));
+    const GuardArgs g = beginGuarded(ctx, r, 0);
     const hipError_t e = kern::padCopyF32(r.stage.as<float>(), r.a.as<float>(), static_cast<int>(r.m),
                                           static_cast<int>(r.k), r.k, static_cast<int>(mp), static_cast<int>(kp),
-                                          ctx->stream);
+                                          ctx->stream, g.word, g.host, g.epoch);
     return e == hipSuccess ? Status::kSuccess : failHip(e, "matmul upload padding (A)");
   }
   const std::size_t mp = roundUp(r.m, kern::kHalfGemmBM);
@@ -60,9 +115,10 @@ Status uploadB(HipContext* ctx, MatMulResident& r, const float* b) {
     LC_TRY(r.stage.ensure(r.k * r.n * sizeof(float)));
     LC_TRY(r.b.ensure(kp * np * sizeof(float)));
     LC_TRY(upload(ctx, r.stage.get(), b, r.k * r.n * sizeof(float)));
+    const GuardArgs g = beginGuarded(ctx, r, 1);
     const hipError_t e = kern::padCopyF32(r.stage.as<float>(), r.b.as<float>(), static_cast<int>(r.k),
                                           static_cast<int>(r.n), r.n, static_cast<int>(kp), static_cast<int>(np),
-                                          ctx->stream);
+                                          ctx->stream, g.word, g.host, g.epoch);
     return e == hipSuccess ? Status::kSuccess : failHip(e, "matmul upload padding (B)");
   }
   const std::size_t np = roundUp(r.n, kern::kHalfGemmBN);
@@ -93,6 +149,10 @@ constexpr VariantInfo kF32Variants[] = {
      "gemm_f32_lds_kernel"},
     {static_cast<int>(kern::GemmF32Variant::kDataParallelBK32), "f32_dp_64x64x32", 64, 64, 32, 8, 2,
      "gemm_f32_lds_kernel"},
+    {static_cast<int>(kern::GemmF32Variant::kSplit64), "f32_split_64x64", 64, 64, 32, 4, 4, "gemm_f32_split_kernel"},
+    {static_cast<int>(kern::GemmF32Variant::kSplit80), "f32_split_80x64", 80, 64, 32, 4, 4, "gemm_f32_split_kernel"},
+    {static_cast<int>(kern::GemmF32Variant::kSplit128), "f32_split_128x128", 128, 128, 32, 4, 1,
+     "gemm_f32_split128_kernel"},
 };
 
 constexpr VariantInfo kHalfVariants[] = {
@@ -154,6 +214,66 @@ bool variantFromEntry(const TuneEntry& e, bool half, std::size_t m, int* variant
   return false;
 }
 
+int cuCount(const HipContext* ctx) {
+  return ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
+}
+
+// The split GEMM keeps 6 bytes more per operand value; past an eighth of the
+// device's memory, or past the kernels' 32-bit offsets along k (160 bytes a k),
+// the fp32 kernels run instead.
+bool splitFits(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t n) {
+  const std::size_t kp = roundUp(k, kern::kF32GemmBK);
+  const std::size_t rows = roundUp(m, kern::kF32GemmBM) + roundUp(n, kern::kF32GemmBN);
+  return kp <= (std::size_t{1} << 23) && 3 * sizeof(uint16_t) * rows * kp <= ctx->props.totalGlobalMem / 8;
+}
+
+bool isSplit(int variant) { return variant >= static_cast<int>(kern::GemmF32Variant::kSplit64); }
+
+// The GEMM of a split variant (its planes made first if they are stale);
+// false when its buffers cannot be had, and nothing was launched.
+bool launchSplitGemm(HipContext* ctx, MatMulResident& r, kern::GemmF32Variant variant, hipError_t* result) {
+  const int M = static_cast<int>(r.m);
+  const int N = static_cast<int>(r.n);
+  const int kp = static_cast<int>(roundUp(r.k, kern::kF32GemmBK));
+  const int np = static_cast<int>(roundUp(r.n, kern::kF32GemmBN));
+  const int mp = static_cast<int>(roundUp(r.m, kern::kF32GemmBM));
+  const int splits = kern::gemmF32SplitCount(variant, M, N, kp, cuCount(ctx));
+  kern::SplitKWork work{nullptr, nullptr};
+  if (splits > 1) {
+    const std::size_t tiles = kern::gemmF32SplitTiles(variant, M, N);
+    if (ctx->splitk_part.ensure(tiles * splits * kern::gemmF32SplitPartFloats(variant) * sizeof(float)) !=
+            Status::kSuccess ||
+        ctx->splitk_counters.ensure(tiles * sizeof(int), true) != Status::kSuccess) {
+      return false;
+    }
+    work = kern::SplitKWork{ctx->splitk_part.as<float>(), ctx->splitk_counters.as<int>()};
+  }
+  const std::size_t na = 3 * static_cast<std::size_t>(mp) * kp;
+  const std::size_t nb = 3 * static_cast<std::size_t>(np) * kp;
+  if (r.planes.size() < (na + nb) * sizeof(uint16_t)) {
+    r.has_planes_a = r.has_planes_b = false;  // growth drops the contents
+  }
+  if (r.planes.ensure((na + nb) * sizeof(uint16_t)) != Status::kSuccess) {
+    return false;
+  }
+  const kern::SplitOperandF32 a{r.a.as<float>(), kp, mp / 16, r.planes.as<uint16_t>()};
+  const kern::SplitOperandF32 b{r.b.as<float>(), np, np / 16, r.planes.as<uint16_t>() + na};
+  if (!r.has_planes_a || !r.has_planes_b) {
+    kern::SplitOperandF32 new_a = a, new_b = b;
+    new_a.src = r.has_planes_a ? nullptr : a.src;
+    new_b.src = r.has_planes_b ? nullptr : b.src;
+    *result = kern::splitPlanesF32(new_a, new_b, kp, ctx->stream);
+    if (*result != hipSuccess) {
+      return true;
+    }
+    r.has_planes_a = r.has_planes_b = true;
+  }
+  const int* words = ctx->guard_words.as<int>() + 2 * r.guard_slot;
+  const kern::SplitGuardF32 guard{words, words + 1, r.epoch_a, r.epoch_b};
+  *result = kern::gemmF32Split(a, b, r.c.as<float>(), M, N, kp, N, guard, work, variant, splits, ctx->stream);
+  return true;
+}
+
 hipError_t launchGemm(HipContext* ctx, MatMulResident& r, int variant) {
   const int M = static_cast<int>(r.m);
   const int K = static_cast<int>(r.k);
@@ -161,8 +281,16 @@ hipError_t launchGemm(HipContext* ctx, MatMulResident& r, int variant) {
   if (!isHalf(r.dtype)) {
     const int kp = static_cast<int>(roundUp(r.k, kern::kF32GemmBK));
     const int np = static_cast<int>(roundUp(r.n, kern::kF32GemmBN));
+    if (isSplit(variant)) {
+      hipError_t e = hipSuccess;
+      if (!knownUnsafe(ctx, r) && splitFits(ctx, r.m, r.k, r.n) &&
+          launchSplitGemm(ctx, r, static_cast<kern::GemmF32Variant>(variant), &e)) {
+        return e;
+      }
+      variant = static_cast<int>(kern::GemmF32Variant::kAuto);
+    }
     // stream-K: one workgroup per CU (a whole-tile grid may hold two per CU)
-    const int groups = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
+    const int groups = cuCount(ctx);
     const bool fresh_fail = ctx->gemm_fail.get() == nullptr;
     if (ctx->gemm_part.ensure(static_cast<std::size_t>(groups) * 4096 * sizeof(float)) != Status::kSuccess ||
         ctx->gemm_flags.ensure(static_cast<std::size_t>(groups) * sizeof(int), true) != Status::kSuccess ||
@@ -241,6 +369,17 @@ Status timeVariants(HipContext* ctx, MatMulResident& r, const std::vector<int>& 
   return Status::kSuccess;
 }
 
+// fp32: the split GEMM where its planes fit, else whole tiles or stream-K.
+int defaultF32Variant(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t n) {
+  const int M = static_cast<int>(m);
+  const int N = static_cast<int>(n);
+  if (!splitFits(ctx, m, k, n)) {
+    return static_cast<int>(kern::gemmF32Choose(M, N, cuCount(ctx)));
+  }
+  return static_cast<int>(
+      kern::gemmF32SplitChoose(M, N, static_cast<int>(roundUp(k, kern::kF32GemmBK)), cuCount(ctx)));
+}
+
 // Settles r.variant for the shape: a tune-cache entry, else (CJ_MATMUL_AUTOTUNE
 // not off) the fastest candidate, else the heuristic; the choice is recorded.
 // CJ_HIP_GEMM_F32 / CJ_HIP_GEMM_TILE (sweep overrides) bypass all of it.
@@ -258,11 +397,17 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
   }
   const int M = static_cast<int>(r.m);
   const int N = static_cast<int>(r.n);
-  const int groups = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
-  int best = half ? static_cast<int>(kern::gemmHalfChoose(M, N)) : static_cast<int>(kern::gemmF32Choose(M, N, groups));
+  int best = half ? static_cast<int>(kern::gemmHalfChoose(M, N)) : defaultF32Variant(ctx, r.m, r.k, r.n);
   std::vector<int> cands;
   if (!half) {
     cands = {static_cast<int>(kern::GemmF32Variant::kDataParallel), static_cast<int>(kern::GemmF32Variant::kStreamK)};
+    if (splitFits(ctx, r.m, r.k, r.n)) {
+      for (const VariantInfo& v : kF32Variants) {
+        if (isSplit(v.variant)) {
+          cands.push_back(v.variant);
+        }
+      }
+    }
   } else if (r.m > 16) {
     for (const VariantInfo& v : kHalfVariants) {
       if (v.variant != static_cast<int>(kern::GemmHalfVariant::kSkinny)) {
@@ -292,6 +437,17 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
   r.variant = best;
   tuneRecord(r.m, r.k, r.n, dtype, arch, entryFor(half, best));
   return Status::kSuccess;
+}
+
+// The variant for a call that uploads an fp32 operand and launches once: the
+// planes of a new operand cost 5 us (256^3) to 12 us (2048^3), more than the
+// split GEMM saves below 2^32 products (1024^3: 6.4 + 16.1 us against 22.3).
+int oneShotVariant(const MatMulResident& r) {
+  const bool stale = !r.has_planes_a || !r.has_planes_b;
+  if (!isHalf(r.dtype) && isSplit(r.variant) && stale && r.m * r.k * r.n < (std::size_t{1} << 32)) {
+    return static_cast<int>(kern::GemmF32Variant::kAuto);
+  }
+  return r.variant;
 }
 
 // Small fp32 calls that upload both operands and download the product (the
@@ -326,11 +482,14 @@ Status matmulQuick(HipContext* ctx, MatMulResident& r, const float* a, const flo
   float* dev = static_cast<float*>(ctx->pinned.device());
   std::memcpy(stage, a, na * sizeof(float));
   std::memcpy(stage + b_at, b, nb * sizeof(float));
+  const GuardArgs ga = beginGuarded(ctx, r, 0);
+  const GuardArgs gb = beginGuarded(ctx, r, 1);
   hipError_t e = kern::padCopyF32(dev, r.a.as<float>(), static_cast<int>(r.m), static_cast<int>(r.k), r.k,
-                                  static_cast<int>(mp), static_cast<int>(kp), ctx->stream);
+                                  static_cast<int>(mp), static_cast<int>(kp), ctx->stream, ga.word, ga.host,
+                                  ga.epoch);
   if (e == hipSuccess) {
     e = kern::padCopyF32(dev + b_at, r.b.as<float>(), static_cast<int>(r.k), static_cast<int>(r.n), r.n,
-                         static_cast<int>(kp), static_cast<int>(np), ctx->stream);
+                         static_cast<int>(kp), static_cast<int>(np), ctx->stream, gb.word, gb.host, gb.epoch);
   }
   if (e != hipSuccess) {
     return failHip(e, "matmul upload padding");
@@ -345,7 +504,7 @@ Status matmulQuick(HipContext* ctx, MatMulResident& r, const float* a, const flo
   unsigned seq = 0;
   LC_TRY(prepareDoneFlag(ctx, &flag_dev, &count_dev, &seq));
   traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, r.m * r.k * r.n);
-  e = launchGemm(ctx, r, r.variant);
+  e = launchGemm(ctx, r, oneShotVariant(r));
   if (e != hipSuccess) {
     return failHip(e, "matmul kernel launch");
   }
@@ -404,9 +563,11 @@ Status matmulResident(HipContext* ctx, MatMulResident& r, std::size_t m, std::si
     LC_TRY(settleVariant(ctx, r));
     r.tuned = true;
   }
+  const bool one_shot = repeat == 1 && policy.download_out && (policy.upload_a || policy.upload_b);
+  const int variant = one_shot ? oneShotVariant(r) : r.variant;
   for (std::size_t i = 0; i < repeat; ++i) {
     traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, hint);
-    const hipError_t e = launchGemm(ctx, r, r.variant);
+    const hipError_t e = launchGemm(ctx, r, variant);
     if (e != hipSuccess) {
       return failHip(e, "matmul kernel launch");
     }
@@ -536,6 +697,7 @@ lcError_t lcMatMulResidentSessionDestroy(lcMatMulResidentSession* s) {
   if (ctx != nullptr) {
     std::lock_guard<std::recursive_mutex> lock(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);
+    releaseGuard(ctx, s->res);
   }
   delete s;
   return LC_SUCCESS;
@@ -651,10 +813,9 @@ lcError_t lcMatMulResidentSessionKernelName(lcMatMulResidentSession* s, char* bu
   const bool half = isHalf(s->dtype);
   int v = s->res.tuned ? s->res.variant : 0;
   if (v == 0) {
-    const int groups = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
-    v = half ? (s->m <= 16 ? static_cast<int>(kern::GemmHalfVariant::kSkinny)
-                           : static_cast<int>(kern::gemmHalfChoose(static_cast<int>(s->m), static_cast<int>(s->n))))
-             : static_cast<int>(kern::gemmF32Choose(static_cast<int>(s->m), static_cast<int>(s->n), groups));
+    v = !half        ? defaultF32Variant(ctx, s->m, s->k, s->n)
+        : s->m <= 16 ? static_cast<int>(kern::GemmHalfVariant::kSkinny)
+                     : static_cast<int>(kern::gemmHalfChoose(static_cast<int>(s->m), static_cast<int>(s->n)));
   }
   std::string text;
   for (const VariantInfo& info : variants(half)) {

@@ -65,6 +65,14 @@ struct MatMulResident {
   // the first launch from the tune cache, an autotune or the heuristic.
   int variant = 0;
   bool tuned = false;
+  // fp32: the bf16 parts of A, then of B (kern::SplitOperandF32), made when a
+  // split GEMM first needs them after an upload.
+  DeviceBuffer planes;
+  bool has_planes_a = false, has_planes_b = false;
+  // fp32: this resident's pair of HipContext::guard_words (-1: none) and the
+  // epochs of the operands' last uploads (0: not guarded).
+  int guard_slot = -1;
+  int epoch_a = 0, epoch_b = 0;
 };
 
 Status matmulResident(HipContext* ctx, MatMulResident& res, std::size_t m, std::size_t k, std::size_t n,

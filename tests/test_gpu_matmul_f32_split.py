@@ -1,0 +1,135 @@
+"""The fp32 GEMM on bf16 planes (csrc/kernels/gemm_f32.hip) vs float64.
+
+Every variant is forced through a seeded tune cache at the sizes where its
+tiles, its k steps or its split of k end: one row or column, one below and one
+above a tile, one k step, fewer steps than waves, more steps than the LDS ring
+has slots, several workgroups a tile.  Bound per element: every output is a sum
+of K exact products; each accumulation rounds (or truncates) to at most 2^-23
+of the running sum of magnitudes, and a value passes through at most
+6 K / 32 + 16 of them, so |error| <= (6 K / 32 + 16) * 2^-23 * (|A| |B|).
+
+Operands that three bf16 values cannot hold exactly (infinities, NaN, tiny and
+huge values) take the fp32 matrix instruction and must give what it gives.
+"""
+import os
+import subprocess
+import sys
+import textwrap
+
+import numpy as np
+import pytest
+
+from gpu_util import note, require_hip
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+VARIANTS = {"f32_split_64x64": "64,64,32,4,4", "f32_split_80x64": "80,64,32,4,4",
+            "f32_split_128x128": "128,128,32,4,1"}
+SHAPES = [(1, 1, 1), (1, 300, 65), (63, 33, 64), (64, 32, 63), (65, 64, 129), (81, 97, 64), (127, 160, 128),
+          (129, 225, 127), (160, 512, 257), (300, 3000, 300), (257, 1056, 513)]
+
+
+@pytest.fixture(scope="module")
+def lc():
+    return require_hip()
+
+
+def _child(code, cwd):
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "lightining-core_amd"))
+    r = subprocess.run([sys.executable, "-u", "-c", textwrap.dedent(code)], cwd=cwd, env=env, capture_output=True,
+                       text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+@pytest.mark.parametrize("name", sorted(VARIANTS))
+def test_split_variants_against_float64(lc, tmp_path, name):
+    cache = tmp_path / "mm.csv"
+    cache.write_text("#lc_tune_cache,matmul,2\n" +
+                     "".join(f"{m},{k},{n},0,gfx950,{name},{VARIANTS[name]}\n" for m, k, n in SHAPES))
+    out = _child(f"""
+        import numpy as np
+        import lightning_core as lc
+        from lightning_core import synth
+        lc.tune_cache_load({str(cache)!r})
+        for m, k, n in {SHAPES!r}:
+            print("[case]", m, k, n, flush=True)
+            a, b = synth.normal((m, k), stream=41), synth.normal((k, n), stream=42)
+            s = lc.MatMulResidentSession(m, k, n)
+            assert s.start_into(a, b) is not None and {name!r} in s.kernel_name()
+            c = s.finish_into().reshape(m, n)
+            again = s.finish_into().reshape(m, n)
+            s.close()
+            assert np.array_equal(c, again)
+            a, b = a.astype(np.float64), b.astype(np.float64)
+            bound = (6 * k / 32 + 16) * 2.0 ** -23 * (np.abs(a) @ np.abs(b))
+            print("WORST", m, k, n, float((np.abs(c - a @ b) / bound).max()), flush=True)
+    """, tmp_path)
+    worst = [line.split()[1:] for line in out.splitlines() if line.startswith("WORST")]
+    assert len(worst) == len(SHAPES)
+    for m, k, n, share in worst:
+        note(f"[parity] {name} {m}x{k}x{n}: {float(share):.3f} of the bound")
+        assert float(share) <= 1.0
+
+
+@pytest.mark.parametrize("m,k,n", [(70, 96, 130), (200, 512, 300), (2048, 1024, 2048)])
+@pytest.mark.parametrize("what", ["nan", "inf", "tiny", "huge", "lowest", "zero"])
+def test_operands_outside_the_split(lc, m, k, n, what):
+    rng = np.random.default_rng(7)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, n), dtype=np.float32)
+    if what == "nan":
+        a[m // 2, k // 3] = np.nan
+    elif what == "inf":
+        b[k // 3, n // 2] = -np.inf
+    elif what == "tiny":  # below 2^-100, where a low part would leave bf16's range
+        a *= np.float32(1e-34)
+        b *= np.float32(1e30)
+    elif what == "huge":
+        a *= np.float32(1e19)
+        b *= np.float32(1e15)
+    elif what == "lowest":
+        a[0] = 0.0
+        a[0, k // 2] = np.finfo(np.float32).min  # one product a row: no partial sum overflows on the way
+    else:
+        a[:] = 0.0
+    with np.errstate(all="ignore"):
+        a64, b64 = a.astype(np.float64), b.astype(np.float64)
+        ref = a64 @ b64
+        bound = (k + 16) * 2.0 ** -23 * (np.abs(a64) @ np.abs(b64))
+    s = lc.matmul2d_resident_session(a, b)
+    out = s.start_into(a, b)
+    first = s.finish_into(out=out).copy().reshape(m, n)  # the kernel's own check may still decide
+    lc.device_synchronize()
+    later = s.finish_into(out=out).reshape(m, n)  # the host knows
+    s.close()
+    call = lc.matmul2d(a, b)
+    clear = np.isfinite(ref) & (np.abs(ref) + bound < 3.0e38)
+    with np.errstate(all="ignore"):
+        special = np.where(clear, 0.0, ref.astype(np.float32))
+    for got in (first, later, call):
+        edge = ~clear & np.isfinite(ref) & (np.abs(ref) <= np.finfo(np.float32).max + bound)  # may round either way
+        np.testing.assert_array_equal(np.where(clear | edge, 0.0, got), np.where(edge, 0.0, special))
+        assert np.all(np.isfinite(got[clear]))
+        assert np.all(np.abs(got[clear] - ref[clear]) <= bound[clear])
+
+
+def test_guard_follows_each_upload(lc):
+    # A fit operand after an unfit one, and back, on one session.
+    rng = np.random.default_rng(9)
+    m, k, n = 130, 200, 70
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, n), dtype=np.float32)
+    bad = a.copy()
+    bad[3, 5] = np.inf
+    s = lc.MatMulResidentSession(m, k, n)
+    for x in (a, bad, a, bad, bad, a):
+        s.start_into(x, b)
+        got = s.finish_into().reshape(m, n)
+        with np.errstate(all="ignore"):
+            ref = x.astype(np.float64) @ b.astype(np.float64)
+        fin = np.isfinite(ref)
+        assert np.array_equal(fin, np.isfinite(got)) and np.array_equal(got[~fin], ref[~fin].astype(np.float32))
+        assert np.abs(got[fin] - ref[fin]).max() <= 1e-5 * np.abs(ref[fin]).max()
+    s.close()

@@ -333,6 +333,55 @@ Status attentionForwardQuick(HipContext* ctx, AttnResident& res, const AttnShape
 
 }  // namespace
 
+namespace {
+
+// Whether the fp32 forward on bf16 planes serves this problem: not the ones
+// small enough for the 16-query kernel (4 heads of S = 256: 7.5 against 12.6
+// us), nor one head up to S = 2048 at D <= 64, where that kernel and the
+// 32-query kernel's key splits are as fast (S = 2048: 23.2 against 23.4 us).
+// The planes take 4.5 times a tensor's fp32 bytes: at most an eighth of memory.
+bool splitServes(const HipContext* ctx, const AttnShape& sh) {
+  const int S = static_cast<int>(sh.seq_len);
+  const int D = static_cast<int>(sh.head_dim);
+  if (isHalf(sh.dtype) || sh.bh() > 65535 || !kern::attentionF32SplitFits(S, D)) {
+    return false;
+  }
+  if (kern::attentionF32DefaultSplits(static_cast<int>(sh.bh()), S, D) == kern::kAttnF32Q16 ||
+      (sh.bh() == 1 && D <= 64 && S <= 2048)) {
+    return false;
+  }
+  const std::size_t bytes = kern::attentionF32PlanesHalves(static_cast<int>(sh.bh()), S, D) * sizeof(uint16_t);
+  return bytes <= ctx->props.totalGlobalMem / 8;
+}
+
+// Makes the planes of the resident q, k and v if they are stale.  False: they
+// cannot be had, or a value does not fit them as far as the host has seen.
+bool ensurePlanes(HipContext* ctx, AttnResident& res, const AttnShape& sh, hipError_t* e) {
+  const int S = static_cast<int>(sh.seq_len);
+  const int D = static_cast<int>(sh.head_dim);
+  const int bh = static_cast<int>(sh.bh());
+  *e = hipSuccess;
+  if (!res.has_planes) {
+    if (res.planes.ensure(kern::attentionF32PlanesHalves(bh, S, D) * sizeof(uint16_t)) != Status::kSuccess) {
+      return false;
+    }
+    const GuardArgs g = beginGuard(ctx, &res.guard_slot, 0);
+    res.epoch = g.epoch;
+    if (g.epoch == 0) {
+      return false;
+    }
+    *e = kern::attentionF32Planes(res.q.as<float>(), res.k.as<float>(), res.v.as<float>(), res.planes.as<uint16_t>(),
+                                  bh, S, D, g.word, g.host, g.epoch, ctx->stream);
+    if (*e != hipSuccess) {
+      return true;
+    }
+    res.has_planes = true;
+  }
+  return !knownUnfit(ctx, res.guard_slot, 0, res.epoch);
+}
+
+}  // namespace
+
 Status attentionForwardResident(HipContext* ctx, AttnResident& res, const AttnShape& sh, const float* q,
                                 const float* k, const float* v, float* out, const lcAttentionIoPolicy& policy,
                                 std::size_t repeat) {
@@ -355,6 +404,9 @@ Status attentionForwardResident(HipContext* ctx, AttnResident& res, const AttnSh
   if (!sameShape(res.shape, sh)) {
     res.has_q = res.has_k = res.has_v = res.has_out = false;
     res.shape = sh;
+  }
+  if (policy.upload_q || policy.upload_k || policy.upload_v) {
+    res.has_planes = false;
   }
   if ((!policy.upload_q && !res.has_q) || (!policy.upload_k && !res.has_k) || (!policy.upload_v && !res.has_v)) {
     return fail(Status::kInvalidValue, "attention: no resident input for a tensor the policy does not upload");
@@ -385,16 +437,36 @@ Status attentionForwardResident(HipContext* ctx, AttnResident& res, const AttnSh
   const int bh = static_cast<int>(sh.bh());
   const std::size_t hint = sh.seq_len * sh.seq_len * sh.head_dim;
   int splits = 0;  // batched fp32 heads keep the heuristic (the cache keys one head)
-  if (!half && bh == 1 && repeat > 0) {
+  hipError_t planes_error = hipSuccess;
+  const bool planes = repeat > 0 && splitServes(ctx, sh) && ensurePlanes(ctx, res, sh, &planes_error);
+  if (planes_error != hipSuccess) {
+    return failHip(planes_error, "attention operand planes");
+  }
+  const int cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
+  if (planes) {
+    LC_TRY(ensureSplitWs(res, kern::attentionF32SplitWorkFloats(bh, S, D, cus)));
+  }
+  if (!half && !planes && bh == 1 && repeat > 0) {
     LC_TRY(forwardSplits(ctx, res, sh, policy, &splits));
   }
-  if (!half) {
+  if (!half && !planes) {
     LC_TRY(ensureSplitWs(res, kern::attentionF32WorkspaceFloats(bh, S, D, splits)));
   }
   for (std::size_t r = 0; r < repeat; ++r) {
     traceOpDispatch(TraceOp::kAttentionForward, Device::kHIP, Device::kHIP, false, hint);
     hipError_t e;
-    if (!half) {
+    if (planes) {
+      const kern::AttnPlanesF32 in{res.planes.as<uint16_t>(),
+                                   res.planes.as<uint16_t>() + 3 * sh.bh() * roundUp(sh.seq_len, 32) * sh.head_dim,
+                                   res.q.as<float>(),
+                                   res.k.as<float>(),
+                                   res.v.as<float>(),
+                                   ctx->guard_words.as<int>() + 2 * res.guard_slot,
+                                   res.epoch};
+      e = kern::attentionF32Split(in, res.out.as<float>(), bh, S, D, sh.causal, policy.output_scale,
+                                  policy.output_bias, policy.output_relu, res.split_ws.as<float>(),
+                                  res.split_ws.size() / sizeof(float), cus, ctx->stream);
+    } else if (!half) {
       e = kern::attentionF32(res.q.as<float>(), res.k.as<float>(), res.v.as<float>(), res.out.as<float>(), bh, S, D,
                              sh.causal, policy.output_scale, policy.output_bias, policy.output_relu, nullptr,
                              ctx->stream, splits, nullptr, nullptr, 0, res.split_ws.as<float>(),
@@ -447,6 +519,7 @@ Status attentionTrainResident(HipContext* ctx, AttnResident& res, const AttnShap
     res.has_q = res.has_k = res.has_v = res.has_out = res.has_target = false;
     res.shape = sh;
   }
+  res.has_planes = false;  // the step changes v
   if ((!policy.upload_q && !res.has_q) || (!policy.upload_k && !res.has_k) || (!policy.upload_v && !res.has_v) ||
       (!policy.upload_target && !res.has_target)) {
     return fail(Status::kInvalidValue, "attention train step: no resident input for a tensor the policy does not upload");
@@ -773,6 +846,7 @@ lcError_t lcAttentionSessionDestroy(lcAttentionSession* session) {
   if (ctx != nullptr) {
     std::lock_guard<std::recursive_mutex> lock(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);  // no kernel may still use the buffers
+    releaseGuard(ctx, &session->res.guard_slot);
     delete session;
   } else {
     delete session;

@@ -162,6 +162,31 @@ hipError_t attentionF32(const float* q, const float* k, const float* v, float* o
                         unsigned* done_flag = nullptr, unsigned done_seq = 0, float* split_ws = nullptr,
                         size_t split_ws_floats = 0);
 size_t attentionF32WorkspaceFloats(int bh, int S, int D, int splits);
+// The same forward from bf16 planes of q, k and v (attention_f32.hip): D a
+// multiple of 32 up to 128, bh <= 65535.  `planes` holds
+// attentionF32PlanesHalves values; attentionF32Planes fills them and sets the
+// guard words as padCopyF32 does (the kernel then uses the fp32 operands).
+// `ws` holds attentionF32SplitWorkFloats floats (0: none needed).
+struct AttnPlanesF32 {
+  const uint16_t* planes_q;
+  const uint16_t* planes_kv;  // planes_q + 3 * bh * roundup(S, 32) * D
+  const float* q;
+  const float* k;
+  const float* v;
+  const int* guard;
+  int epoch;
+};
+bool attentionF32SplitFits(int S, int D);
+size_t attentionF32PlanesHalves(int bh, int S, int D);
+hipError_t attentionF32Planes(const float* q, const float* k, const float* v, uint16_t* planes, int bh, int S, int D,
+                              int* guard, int* guard_host, int epoch, hipStream_t stream);
+size_t attentionF32SplitWorkFloats(int bh, int S, int D, int cus);
+hipError_t attentionF32Split(const AttnPlanesF32& in, float* out, int bh, int S, int D, bool causal, float post_scale,
+                             float post_bias, int post_relu, float* ws, size_t ws_floats, int cus,
+                             hipStream_t stream);
+// Merges nsplit partials [z][head][S][D] and their (m, l) [z][head][S][2] in ws.
+hipError_t attentionF32Combine(const float* ws, float* out, int bh, int S, int D, int nsplit, float post_scale,
+                               float post_bias, int post_relu, hipStream_t stream);
 // The `splits` value that selects the 16-query fp32 forward kernel
 // (attn_fwd_f32_q16_kernel: 16 waves of 16-key tiles per 16 queries), for
 // problems too small to fill the GPU.  Needs D <= 64, D % 4 == 0 and 16-byte

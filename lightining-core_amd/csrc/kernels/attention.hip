@@ -2206,6 +2206,14 @@ hipError_t attentionF32(const float* q, const float* k, const float* v, float* o
   return hipGetLastError();
 }
 
+hipError_t attentionF32Combine(const float* ws, float* out, int bh, int S, int D, int nsplit, float post_scale,
+                               float post_bias, int post_relu, hipStream_t stream) {
+  const int rows = bh * S;
+  hipLaunchKernelGGL(attn_split_combine_kernel, dim3((rows + 3) / 4), dim3(256), 0, stream, ws, out, nullptr, rows, D,
+                     nsplit, post_scale, post_bias, post_relu, DoneFlag{});
+  return hipGetLastError();
+}
+
 bool convAttentionStagesInputs(int batch, int cin, int h, int wd, int cout, int kh, int kw, int sh, int sw, int ph,
                                int pw) {
   const int oh = (h + 2 * ph - kh) / sh + 1;

@@ -27,20 +27,7 @@
 
 namespace lchip {
 
-namespace {
-
-// fp32 operands are scanned while they are padded (`which` 0: A, 1: B): the
-// words of the split GEMM's guard, and the epoch of this copy (every copy has
-// a new one, so the words are never cleared).
-struct GuardArgs {
-  int* word;  // null: not guarded
-  int* host;  // device alias
-  int epoch;
-};
-GuardArgs beginGuarded(HipContext* ctx, MatMulResident& r, int which) {
-  int& epoch = which == 0 ? r.epoch_a : r.epoch_b;
-  epoch = 0;
-  (which == 0 ? r.has_planes_a : r.has_planes_b) = false;
+GuardArgs beginGuard(HipContext* ctx, int* slot, int which) {
   if (ctx->guard_host.get() == nullptr) {
     const std::size_t bytes = 2 * kGuardSlots * sizeof(int);
     if (ctx->guard_words.ensure(bytes, true) != Status::kSuccess ||
@@ -52,34 +39,41 @@ GuardArgs beginGuarded(HipContext* ctx, MatMulResident& r, int which) {
       ctx->guard_free.push_back(i);
     }
   }
-  if (r.guard_slot < 0 && !ctx->guard_free.empty()) {
-    r.guard_slot = ctx->guard_free.back();
+  if (*slot < 0 && !ctx->guard_free.empty()) {
+    *slot = ctx->guard_free.back();
     ctx->guard_free.pop_back();
   }
-  if (r.guard_slot < 0 || ctx->guard_epoch == INT_MAX) {
+  if (*slot < 0 || ctx->guard_epoch == INT_MAX) {
     return GuardArgs{nullptr, nullptr, 0};
   }
-  epoch = ++ctx->guard_epoch;
-  const int at = 2 * r.guard_slot + which;
-  return GuardArgs{ctx->guard_words.as<int>() + at, static_cast<int*>(ctx->guard_host.device()) + at, epoch};
+  const int at = 2 * *slot + which;
+  return GuardArgs{ctx->guard_words.as<int>() + at, static_cast<int*>(ctx->guard_host.device()) + at,
+                   ++ctx->guard_epoch};
 }
 
-void releaseGuard(HipContext* ctx, MatMulResident& r) {
-  if (r.guard_slot >= 0) {
-    ctx->guard_free.push_back(r.guard_slot);
-    r.guard_slot = -1;
+void releaseGuard(HipContext* ctx, int* slot) {
+  if (*slot >= 0) {
+    ctx->guard_free.push_back(*slot);
+    *slot = -1;
   }
 }
 
-// Whether an operand was not guarded, or the host has already seen that it is
-// unfit for the split (its upload has finished; until then the kernel's own
-// check decides).
+bool knownUnfit(const HipContext* ctx, int slot, int which, int epoch) {
+  return epoch == 0 || static_cast<const volatile int*>(ctx->guard_host.get())[2 * slot + which] == epoch;
+}
+
+namespace {
+
+// The guard of an fp32 operand about to be uploaded (`which` 0: A, 1: B).
+GuardArgs beginUpload(HipContext* ctx, MatMulResident& r, int which) {
+  const GuardArgs g = beginGuard(ctx, &r.guard_slot, which);
+  (which == 0 ? r.epoch_a : r.epoch_b) = g.epoch;
+  (which == 0 ? r.has_planes_a : r.has_planes_b) = false;
+  return g;
+}
+
 bool knownUnsafe(const HipContext* ctx, const MatMulResident& r) {
-  if (r.epoch_a == 0 || r.epoch_b == 0) {
-    return true;
-  }
-  const volatile int* w = static_cast<const volatile int*>(ctx->guard_host.get()) + 2 * r.guard_slot;
-  return w[0] == r.epoch_a || w[1] == r.epoch_b;
+  return knownUnfit(ctx, r.guard_slot, 0, r.epoch_a) || knownUnfit(ctx, r.guard_slot, 1, r.epoch_b);
 }
 
 Status uploadA(HipContext* ctx, MatMulResident& r, const float* a) {
@@ -90,7 +84,7 @@ Status uploadA(HipContext* ctx, MatMulResident& r, const float* a) {
     LC_TRY(r.stage.ensure(r.m * r.k * sizeof(float)));
     LC_TRY(r.a.ensure(mp * kp * sizeof(float)));
     LC_TRY(upload(ctx, r.stage.get(), a, r.m * r.k * sizeof(float)));
-    const GuardArgs g = beginGuarded(ctx, r, 0);
+    const GuardArgs g = beginUpload(ctx, r, 0);
     const hipError_t e = kern::padCopyF32(r.stage.as<float>(), r.a.as<float>(), static_cast<int>(r.m),
                                           static_cast<int>(r.k), r.k, static_cast<int>(mp), static_cast<int>(kp),
                                           ctx->stream, g.word, g.host, g.epoch);
@@ -115,7 +109,7 @@ Status uploadB(HipContext* ctx, MatMulResident& r, const float* b) {
     LC_TRY(r.stage.ensure(r.k * r.n * sizeof(float)));
     LC_TRY(r.b.ensure(kp * np * sizeof(float)));
     LC_TRY(upload(ctx, r.stage.get(), b, r.k * r.n * sizeof(float)));
-    const GuardArgs g = beginGuarded(ctx, r, 1);
+    const GuardArgs g = beginUpload(ctx, r, 1);
     const hipError_t e = kern::padCopyF32(r.stage.as<float>(), r.b.as<float>(), static_cast<int>(r.k),
                                           static_cast<int>(r.n), r.n, static_cast<int>(kp), static_cast<int>(np),
                                           ctx->stream, g.word, g.host, g.epoch);
@@ -482,8 +476,8 @@ Status matmulQuick(HipContext* ctx, MatMulResident& r, const float* a, const flo
   float* dev = static_cast<float*>(ctx->pinned.device());
   std::memcpy(stage, a, na * sizeof(float));
   std::memcpy(stage + b_at, b, nb * sizeof(float));
-  const GuardArgs ga = beginGuarded(ctx, r, 0);
-  const GuardArgs gb = beginGuarded(ctx, r, 1);
+  const GuardArgs ga = beginUpload(ctx, r, 0);
+  const GuardArgs gb = beginUpload(ctx, r, 1);
   hipError_t e = kern::padCopyF32(dev, r.a.as<float>(), static_cast<int>(r.m), static_cast<int>(r.k), r.k,
                                   static_cast<int>(mp), static_cast<int>(kp), ctx->stream, ga.word, ga.host,
                                   ga.epoch);
@@ -697,7 +691,7 @@ lcError_t lcMatMulResidentSessionDestroy(lcMatMulResidentSession* s) {
   if (ctx != nullptr) {
     std::lock_guard<std::recursive_mutex> lock(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);
-    releaseGuard(ctx, s->res);
+    releaseGuard(ctx, &s->res.guard_slot);
   }
   delete s;
   return LC_SUCCESS;

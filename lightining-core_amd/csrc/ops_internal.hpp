@@ -10,6 +10,22 @@ inline bool isHalf(lcDataType t) { return t == LC_DTYPE_BF16 || t == LC_DTYPE_F1
 inline kern::Half halfOf(lcDataType t) { return t == LC_DTYPE_F16 ? kern::Half::kF16 : kern::Half::kBF16; }
 inline bool validDtype(lcDataType t) { return t == LC_DTYPE_F32 || t == LC_DTYPE_BF16 || t == LC_DTYPE_F16; }
 
+// fp32 operands are scanned while they are copied for kernels that hold a
+// value as three bf16 parts (kern::SplitGuardF32): a resident holds a slot of
+// HipContext::guard_words, two words; every copy has a new epoch, so words are
+// never cleared.  beginGuard takes a slot if the resident has none; epoch 0:
+// not guarded (no slot left), such an operand counts as unfit.
+struct GuardArgs {
+  int* word;
+  int* host;  // device alias
+  int epoch;
+};
+GuardArgs beginGuard(HipContext* ctx, int* slot, int which);
+void releaseGuard(HipContext* ctx, int* slot);
+// Whether the operand is unfit as far as the host has seen (its copy may not
+// have run yet: the kernel's own check decides then).
+bool knownUnfit(const HipContext* ctx, int slot, int which, int epoch);
+
 // Shape of an attention problem: batch*heads independent [S, D] problems.
 struct AttnShape {
   std::size_t batch = 1;
@@ -34,6 +50,12 @@ struct AttnResident {
   DeviceBuffer target, stats, loss;
   DeviceBuffer v_scratch;  // the train step's dV autotune runs on a copy of V
   DeviceBuffer split_ws;   // partials of the fp32 forward's key splits
+  // fp32: the bf16 parts of q, k and v (kern::AttnPlanesF32), made when the
+  // forward first needs them after one of the three has changed.
+  DeviceBuffer planes;
+  bool has_planes = false;
+  int guard_slot = -1;
+  int epoch = 0;
   bool has_q = false, has_k = false, has_v = false, has_out = false, has_target = false;
 };
 
@@ -69,8 +91,8 @@ struct MatMulResident {
   // split GEMM first needs them after an upload.
   DeviceBuffer planes;
   bool has_planes_a = false, has_planes_b = false;
-  // fp32: this resident's pair of HipContext::guard_words (-1: none) and the
-  // epochs of the operands' last uploads (0: not guarded).
+  // fp32: this resident's guard slot (-1: none) and the epochs of the
+  // operands' last uploads (0: not guarded).
   int guard_slot = -1;
   int epoch_a = 0, epoch_b = 0;
 };

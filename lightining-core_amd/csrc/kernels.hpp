@@ -264,7 +264,7 @@ hipError_t convertTransposePad(const float* src, uint16_t* dst, int batch, int r
 // (CJ_HIP_GEMM_TILE=w4h|w4r|w4|w4d|lds|big8|big4|mid|small overrides it).
 enum class GemmHalfVariant {
   kAuto = 0, kLds = 1, kBig8 = 2, kBig4 = 3, kMid = 4, kSmall = 5, kSkinny = 6, kW4 = 7, kW4D = 8, kW4R = 9,
-  kW4H = 10
+  kW4H = 10, kR128 = 11, kR96 = 12, kR64x128 = 13, kR64 = 14, kR32 = 15
 };
 GemmHalfVariant gemmHalfChoose(int M, int N);
 // Workspace of the skinny GEMM's split-K: partial tiles (max_splits x
@@ -285,6 +285,16 @@ int skinnySplits(int N, int K, int cus);
 hipError_t gemmHalfTN(const uint16_t* A, const uint16_t* Bt, float* C, int M, int N, int K, int lda, int ldb,
                       int ldc, Half t, GemmHalfVariant variant, hipStream_t stream,
                       const SkinnyWork* skinny = nullptr);
+// The same product by the kernel of gemm_half.hip, for problems with fewer
+// than a 256x256 tile per CU: variants kR128 (128 x 128 tiles), kR96 (96 x
+// 128), kR64x128, kR64 (64 x 64) and kR32 (32 x 64).
+inline bool gemmHalfR4Fits(long long lda, long long ldb) {
+  return 256LL * lda * 2 < (1LL << 31) && 256LL * ldb * 2 < (1LL << 31);
+}
+inline bool isR4(GemmHalfVariant v) { return v >= GemmHalfVariant::kR128; }
+GemmHalfVariant gemmHalfR4Choose(int M, int N, int K, int cus);
+hipError_t gemmHalfR4(const uint16_t* A, const uint16_t* Bt, float* C, int M, int N, int K, int lda, int ldb, int ldc,
+                      Half t, GemmHalfVariant variant, hipStream_t stream);
 // Same GEMM with a 16-bit output (optionally ReLU).
 hipError_t gemmHalfTNHalfOut(const uint16_t* A, const uint16_t* Bt, uint16_t* C, int M, int N, int K, int lda,
                              int ldb, int ldc, int relu, Half t, hipStream_t stream);

@@ -14,12 +14,12 @@
 #include <type_traits>
 
 #include "../kernels.hpp"
+#include "gemm_tiles.hpp"
 #include "kcommon.hpp"
 
 namespace lchip::k {
 
 using kern::SplitGuardF32;
-using kern::SplitKWork;
 using kern::SplitOperandF32;
 
 // ---------------------------------------------------------------------------
@@ -93,24 +93,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_at(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00027000);
 }
 
-// Tile of workgroup w: w runs on XCD w % 8, and each XCD gets a contiguous
-// range of an order that walks groups of GROUP tile rows.
-template <int GROUP>
-__device__ __forceinline__ void tile_origin(int tiles_m, int tiles_n, int tile_h, int tile_w, int& bm, int& bn) {
-  const int full = (tiles_m * tiles_n) & ~7;
-  int pid = blockIdx.x;
-  if (pid < full) {
-    pid = (pid & 7) * (full >> 3) + (pid >> 3);
-  }
-  const int group_size = GROUP * tiles_n;
-  const int group = pid / group_size;
-  const int first_m = group * GROUP;
-  const int gm = min(tiles_m - first_m, GROUP);
-  const int in_group = pid - group * group_size;
-  bm = (first_m + in_group % gm) * tile_h;
-  bn = (in_group / gm) * tile_w;
-}
-
 // The step of wave-uniform index t of a 16 R x 64 block on the fp32 matrix
 // instruction, for operands the planes cannot hold.
 template <int R>
@@ -169,82 +151,6 @@ __device__ __forceinline__ void add_acc(floatx4 (&acc)[R][4], floatx4 (&low)[R][
       acc[b][j] += low[b][j];
     }
   }
-}
-
-// C[m][n .. n + 3] = v, masked to [M, N].
-__device__ __forceinline__ void store_c4(float* C, int ldc, int m, int n, int M, int N, int vec4, floatx4 v) {
-  if (m >= M) {
-    return;
-  }
-  float* p = C + static_cast<size_t>(m) * ldc + n;
-  if (vec4 && n + 3 < N) {
-    *reinterpret_cast<floatx4*>(p) = v;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if (n + i < N) {
-        p[i] = v[i];
-      }
-    }
-  }
-}
-
-// The sum of acc over the gridDim.y workgroups of a tile, in k order, in the
-// workgroup that finishes last (false in the others); every wave sums its own
-// R row blocks.  Partials move with device-scope (sc1) stores and loads,
-// coherent across the XCDs' L2s; the vmcnt wait orders the stores before the
-// counter bump.  No workgroup waits for another, and the last one leaves the
-// tile's counter at zero.
-template <int R>
-__device__ __forceinline__ bool sum_splits(const SplitKWork& work, int lane, int wave, int* last,
-                                           floatx4 (&acc)[R][4]) {
-  const size_t tile = blockIdx.x;
-  const int splits = gridDim.y;
-  auto part = [&](int y, int b, int j) {
-    return work.part + (((tile * splits + y) * 4 + wave) * R + b) * 1024 + j * 256 + lane;
-  };
-#pragma unroll
-  for (int b = 0; b < R; ++b) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        __hip_atomic_store(part(blockIdx.y, b, j) + i * 64, acc[b][j][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-  }
-  wait_vmcnt<0>();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    *last = __hip_atomic_fetch_add(work.counters + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1;
-  }
-  __syncthreads();
-  if (*last == 0) {
-    return false;
-  }
-#pragma unroll
-  for (int b = 0; b < R; ++b) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      acc[b][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
-  }
-  for (int y = 0; y < splits; ++y) {
-#pragma unroll
-    for (int b = 0; b < R; ++b) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          acc[b][j][i] += __hip_atomic_load(part(y, b, j) + i * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    }
-  }
-  if (threadIdx.x == 0) {
-    __hip_atomic_store(work.counters + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  return true;
 }
 
 // The six products (plane of A, plane of B; 0 = h), the small ones first.

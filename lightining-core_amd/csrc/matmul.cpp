@@ -163,6 +163,11 @@ constexpr VariantInfo kHalfVariants[] = {
     {static_cast<int>(kern::GemmHalfVariant::kBig4), "half_big4_256x256", 256, 256, 64, 4, 1, "gemm_half_tn_kernel"},
     {static_cast<int>(kern::GemmHalfVariant::kMid), "half_mid_128x128", 128, 128, 64, 4, 1, "gemm_half_tn_kernel"},
     {static_cast<int>(kern::GemmHalfVariant::kSmall), "half_small_64x64", 64, 64, 64, 4, 1, "gemm_half_tn_kernel"},
+    {static_cast<int>(kern::GemmHalfVariant::kR128), "half_r4_128x128", 128, 128, 64, 4, 1, "gemm_half_tn_r4_kernel"},
+    {static_cast<int>(kern::GemmHalfVariant::kR96), "half_r4_96x128", 96, 128, 64, 4, 1, "gemm_half_tn_r4_kernel"},
+    {static_cast<int>(kern::GemmHalfVariant::kR64x128), "half_r4_64x128", 64, 128, 64, 4, 1, "gemm_half_tn_r4_kernel"},
+    {static_cast<int>(kern::GemmHalfVariant::kR64), "half_r4_64x64", 64, 64, 64, 4, 1, "gemm_half_tn_r4_kernel"},
+    {static_cast<int>(kern::GemmHalfVariant::kR32), "half_r4_32x64", 32, 64, 64, 4, 1, "gemm_half_tn_r4_kernel"},
     {static_cast<int>(kern::GemmHalfVariant::kSkinny), "half_skinny_16x64", 16, 64, 256, 8, 2, "gemm_skinny_kernel"},
 };
 
@@ -194,11 +199,15 @@ TuneEntry entryFor(bool half, int variant) {
 }
 
 // A cached entry names a variant this shape can run (else it is ignored).
-bool variantFromEntry(const TuneEntry& e, bool half, std::size_t m, int* variant) {
+bool variantFromEntry(const TuneEntry& e, bool half, std::size_t m, std::size_t k, int* variant) {
+  const long long k_pad = static_cast<long long>(roundUp(k, kern::kHalfGemmBK));
   for (const VariantInfo& v : variants(half)) {
     if (e.kernel == v.name) {
       const bool skinny = v.variant == static_cast<int>(kern::GemmHalfVariant::kSkinny);
       if (half && skinny != (m <= 16)) {
+        return false;
+      }
+      if (half && kern::isR4(static_cast<kern::GemmHalfVariant>(v.variant)) && !kern::gemmHalfR4Fits(k_pad, k_pad)) {
         return false;
       }
       *variant = v.variant;
@@ -303,6 +312,10 @@ hipError_t launchGemm(HipContext* ctx, MatMulResident& r, int variant) {
                                static_cast<kern::GemmF32Variant>(variant), ctx->stream);
   }
   const int kp = static_cast<int>(roundUp(r.k, kern::kHalfGemmBK));
+  if (kern::isR4(static_cast<kern::GemmHalfVariant>(variant))) {
+    return kern::gemmHalfR4(r.a.as<uint16_t>(), r.b.as<uint16_t>(), r.c.as<float>(), M, N, kp, kp, kp, N,
+                            halfOf(r.dtype), static_cast<kern::GemmHalfVariant>(variant), ctx->stream);
+  }
   kern::SkinnyWork skinny{nullptr, nullptr, 0, 0, 0};
   if (M <= 16) {
     const int tiles = static_cast<int>(roundUp(r.n, 64) / 64);
@@ -374,6 +387,19 @@ int defaultF32Variant(const HipContext* ctx, std::size_t m, std::size_t k, std::
       kern::gemmF32SplitChoose(M, N, static_cast<int>(roundUp(k, kern::kF32GemmBK)), cuCount(ctx)));
 }
 
+// 16 bits: the skinny kernel up to 16 rows, 256x256 tiles while there is one
+// per CU, else the smaller tiles of gemm_half.hip (within its 32-bit offsets).
+int defaultHalfVariant(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t n) {
+  const int M = static_cast<int>(m);
+  const int N = static_cast<int>(n);
+  const kern::GemmHalfVariant v = kern::gemmHalfChoose(M, N);
+  const int kp = static_cast<int>(roundUp(k, kern::kHalfGemmBK));
+  if ((v == kern::GemmHalfVariant::kMid || v == kern::GemmHalfVariant::kSmall) && kern::gemmHalfR4Fits(kp, kp)) {
+    return static_cast<int>(kern::gemmHalfR4Choose(M, N, kp, cuCount(ctx)));
+  }
+  return static_cast<int>(v);
+}
+
 // Settles r.variant for the shape: a tune-cache entry, else (CJ_MATMUL_AUTOTUNE
 // not off) the fastest candidate, else the heuristic; the choice is recorded.
 // CJ_HIP_GEMM_F32 / CJ_HIP_GEMM_TILE (sweep overrides) bypass all of it.
@@ -386,12 +412,10 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
   const std::string arch = baseArch(ctx);
   const int dtype = static_cast<int>(r.dtype);
   TuneEntry known;
-  if (tuneLookup(r.m, r.k, r.n, dtype, arch, &known) && variantFromEntry(known, half, r.m, &r.variant)) {
+  if (tuneLookup(r.m, r.k, r.n, dtype, arch, &known) && variantFromEntry(known, half, r.m, r.k, &r.variant)) {
     return Status::kSuccess;
   }
-  const int M = static_cast<int>(r.m);
-  const int N = static_cast<int>(r.n);
-  int best = half ? static_cast<int>(kern::gemmHalfChoose(M, N)) : defaultF32Variant(ctx, r.m, r.k, r.n);
+  int best = half ? defaultHalfVariant(ctx, r.m, r.k, r.n) : defaultF32Variant(ctx, r.m, r.k, r.n);
   std::vector<int> cands;
   if (!half) {
     cands = {static_cast<int>(kern::GemmF32Variant::kDataParallel), static_cast<int>(kern::GemmF32Variant::kStreamK)};
@@ -402,9 +426,12 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
         }
       }
     }
-  } else if (r.m > 16) {
+  } else if (r.m > 16 && kern::gemmHalfR4Fits(roundUp(r.k, kern::kHalfGemmBK), roundUp(r.k, kern::kHalfGemmBK))) {
+    // The other kernels were slower than one of these at every shape tried;
+    // they stay for a tune cache or CJ_HIP_GEMM_TILE that names them.
+    cands = {static_cast<int>(kern::GemmHalfVariant::kW4H)};
     for (const VariantInfo& v : kHalfVariants) {
-      if (v.variant != static_cast<int>(kern::GemmHalfVariant::kSkinny)) {
+      if (kern::isR4(static_cast<kern::GemmHalfVariant>(v.variant))) {
         cands.push_back(v.variant);
       }
     }
@@ -807,9 +834,7 @@ lcError_t lcMatMulResidentSessionKernelName(lcMatMulResidentSession* s, char* bu
   const bool half = isHalf(s->dtype);
   int v = s->res.tuned ? s->res.variant : 0;
   if (v == 0) {
-    v = !half        ? defaultF32Variant(ctx, s->m, s->k, s->n)
-        : s->m <= 16 ? static_cast<int>(kern::GemmHalfVariant::kSkinny)
-                     : static_cast<int>(kern::gemmHalfChoose(static_cast<int>(s->m), static_cast<int>(s->n)));
+    v = half ? defaultHalfVariant(ctx, s->m, s->k, s->n) : defaultF32Variant(ctx, s->m, s->k, s->n);
   }
   std::string text;
   for (const VariantInfo& info : variants(half)) {

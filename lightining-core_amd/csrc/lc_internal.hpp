@@ -170,7 +170,10 @@ bool hipAvailable();
 // gfx950 device is visible).
 HipContext* hipContext(Status* st);
 
-// Upload / download on the context stream (pageable host memory).
+// Upload / download on the context stream (pageable host memory).  When they
+// return, an upload's source may be reused and a download's result of
+// kStagedCopyMin bytes or more is in place (smaller ones after a stream sync).
+constexpr std::size_t kStagedCopyMin = std::size_t{32} << 20;
 Status upload(HipContext* ctx, void* dst, const void* src, std::size_t bytes);
 Status download(HipContext* ctx, void* dst, const void* src, std::size_t bytes);
 // Synchronises the backend stream, then reports a failure a kernel recorded

@@ -246,16 +246,6 @@ void PinnedBuffer::reset() {
   bytes_ = 0;
 }
 
-Status upload(HipContext* ctx, void* dst, const void* src, std::size_t bytes) {
-  LC_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
-  return Status::kSuccess;
-}
-
-Status download(HipContext* ctx, void* dst, const void* src, std::size_t bytes) {
-  LC_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  return Status::kSuccess;
-}
-
 namespace {
 // Bookkeeping after the stream has drained: in-flight counts restart, and a
 // failure a kernel recorded since the last sync becomes an error.

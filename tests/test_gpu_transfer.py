@@ -1,0 +1,72 @@
+"""Copies of large host arrays through the pinned ring (csrc/transfer.cpp).
+
+A MatMul of small whole numbers is exact in fp32, so an array that came up or
+went down in the wrong place shows in the result.  Operand and result have the
+same number of bytes: just below the line where the ring takes over, on it, one
+row above, a ring's worth and a remainder, and one with partly filled chunks.
+"""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+from gpu_util import require_hip
+
+pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def lc():
+    return require_hip()
+
+
+def product(lc, rows, seed, out=None):
+    rng = np.random.default_rng(seed)
+    a = rng.integers(-8, 9, (rows, 4)).astype(np.float32)
+    b = rng.integers(-8, 9, (4, 4)).astype(np.float32)
+    out = np.empty((rows, 4), np.float32) if out is None else out
+    out[:] = np.nan
+    s = lc.MatMulResidentSession(rows, 4, 4, "f32")
+    s.start_into(a, b, out)
+    s.finish_into(out=out)
+    s.close()
+    return out, a @ b
+
+
+@pytest.mark.parametrize("rows", [2 * MIB - 1, 2 * MIB, 2 * MIB + 1, 3 * MIB + 12345, 4 * MIB + 65537])
+def test_large_arrays_arrive_whole(lc, rows):
+    for seed in range(2):  # new inputs in the same ring
+        got, want = product(lc, rows, seed)
+        assert np.array_equal(got, want)
+
+
+def test_two_threads_copy_at_once(lc):
+    results = {}
+
+    def work(i):
+        results[i] = product(lc, 2 * MIB + 777 * i, 10 + i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(results) == 2
+    for got, want in results.values():
+        assert np.array_equal(got, want)
+
+
+def test_pinned_result_buffer(lc):
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime the backend has loaded
+    rows = 2 * MIB + 5
+    ptr = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(ptr), ctypes.c_size_t(rows * 16), 0) == 0
+    out = np.ctypeslib.as_array(ctypes.cast(ptr, ctypes.POINTER(ctypes.c_float)), (rows, 4))
+    got, want = product(lc, rows, 3, out)
+    same = np.array_equal(got, want)
+    del got, out
+    assert hip.hipHostFree(ptr) == 0
+    assert same

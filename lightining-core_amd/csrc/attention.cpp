@@ -474,7 +474,7 @@ Status attentionForwardResident(HipContext* ctx, AttnResident& res, const AttnSh
     } else {
       e = kern::attentionHalf(res.q.as<uint16_t>(), res.k.as<uint16_t>(), res.v.as<uint16_t>(), res.out.as<float>(),
                               nullptr, static_cast<int>(sh.heads), bh, S, static_cast<int>(sh.sPad()), D, sh.causal,
-                              halfOf(sh.dtype), ctx->stream);
+                              halfOf(sh.dtype), cus, ctx->stream);
       if (e == hipSuccess && !postIsIdentity(policy)) {
         e = kern::postprocessF32(res.out.as<float>(), n, policy.output_scale, policy.output_bias, policy.output_relu,
                                  ctx->stream);

@@ -364,7 +364,7 @@ Status vitForwardDevice(HipContext* ctx, lcVitBlockSession* s) {
   traceOpDispatch(TraceOp::kAttentionForward, Device::kHIP, Device::kHIP, false, s->T * s->T * s->Dh);
   e = kern::attentionHalf(s->q16.as<uint16_t>(), s->k16.as<uint16_t>(), s->vt16.as<uint16_t>(), nullptr,
                           s->attn16.as<uint16_t>(), H, B * H, T, static_cast<int>(s->S_pad), static_cast<int>(s->Dh),
-                          false, ht, ctx->stream);
+                          false, ht, ctx->props.multiProcessorCount, ctx->stream);
   if (e != hipSuccess) {
     return failHip(e, "vit attention launch");
   }

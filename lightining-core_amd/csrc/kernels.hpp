@@ -325,7 +325,7 @@ hipError_t outProjectGemm(const uint16_t* attn, const uint16_t* Wo_t, float* out
 // rows out[(b*S + s), h*D + d] of a [B*S, H*D] matrix (heads = H).
 hipError_t attentionHalf(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out_f32,
                          uint16_t* out_heads_concat, int heads, int bh, int S, int S_pad, int D, bool causal, Half t,
-                         hipStream_t stream);
+                         int cus, hipStream_t stream);
 
 // ViT: QKV projection of each (image, head) fused with its attention
 // (vit_qkv_attn_kernel); tokens [B*T][E], Wqkv_t [3E][E], output

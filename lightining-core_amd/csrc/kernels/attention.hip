@@ -1388,6 +1388,15 @@ struct HalfAttnWave {
   // VALU work, then tile j's O^T += V^T . P^T (V^T tile at vs).
   __device__ __forceinline__ void step(int j, const uint16_t* ksn, const uint16_t* vs, floatx16 (&s_cur)[2],
                                        floatx16 (&s_nxt)[2]) {
+    u32x4 pb[4];
+    probabilities(j, ksn, s_cur, s_nxt, pb);
+    values(vs, pb);
+  }
+
+  // step's first half: tile j's probabilities (packed to pb) and the next
+  // tile's scores.
+  __device__ __forceinline__ void probabilities(int j, const uint16_t* ksn, floatx16 (&s_cur)[2],
+                                                floatx16 (&s_nxt)[2], u32x4 (&pb)[4]) {
       const int j0 = j * KT;
       if ((j0 + KT > S) || (causal && j0 + KT - 1 > q0)) {
         // key = j0 + 8*half + off with off a compile-time constant per register;
@@ -1417,10 +1426,11 @@ struct HalfAttnWave {
       // unchanged by a shift.
       const bool valid = mt > 0.5f * kMaskValue;
       const bool shift = valid && (!started || mt > 8.0f);
-      started = started || valid;
       if (__any(shift)) {
         const float sh = shift ? mt : 0.0f;
-        const float alpha = fast_exp2(-sh);
+        // nothing to rescale at the first shift, which may go down (exp2(-sh)
+        // would overflow for scores below -128)
+        const float alpha = started ? fast_exp2(-sh) : 1.0f;
         m_run += sh;
         l_run *= alpha;
   #pragma unroll
@@ -1438,7 +1448,8 @@ struct HalfAttnWave {
           }
         }
       }
-      // Phase 1: the 32 exponentials of this lane, packed to 16-bit pairs as
+      started = started || valid;
+      // The 32 exponentials of this lane, packed to 16-bit pairs as
       // they come, with the next tile's 2*QS QK^T MFMAs issued between them
       // (EPM exponentials per MFMA, K fragments read two MFMAs ahead).  The
       // sched_barrier after each group keeps this order: an MFMA runs for 32
@@ -1451,7 +1462,6 @@ struct HalfAttnWave {
         negm[i] = -m_run;
       }
       float ls = 0.0f;
-      u32x4 pb[4];
       auto kfrag = [&](int g) {
         const int kt = g / QS;
         const int s = g - kt * QS;
@@ -1485,7 +1495,10 @@ struct HalfAttnWave {
         __builtin_amdgcn_sched_barrier(0);
       }
       l_run += ls;
-      // Phase 2: O^T += V^T . P^T, V^T fragments read two MFMAs ahead.
+  }
+
+  // step's second half: O^T += V^T . P^T, V^T fragments read two MFMAs ahead.
+  __device__ __forceinline__ void values(const uint16_t* vs, const u32x4 (&pb)[4]) {
       auto vfrag = [&](int g) {
         const int ks2 = g / DT;
         const int t = g - ks2 * DT;
@@ -1652,6 +1665,177 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_half_kernel(const uint16_t* _
     }
   }
   w.store(O, Ocat, bh, heads);
+}
+
+// ---------------------------------------------------------------------------
+// 16-bit attention of problems with too few 128-query blocks to fill the chip:
+// 32 queries per workgroup, and KS waves that share the keys, wave w taking the
+// 64-key tiles w, w + KS, ...  A wave's K and V^T tiles are its own (one LDS
+// buffer each, refilled as soon as its half of the step has read it), so the
+// loop has no barrier; the KS states merge through LDS.  Bound: the serial
+// chain of a wave's tiles (KS times shorter than attn_fwd_half_kernel's, on
+// four times as many workgroups), then launch and merge.  Measured with KS = 4,
+// bf16 (us, attn_fwd_half_kernel -> this): one head of 4096x128 73.3 -> 28.8,
+// of 1400x64 20.6 -> 9.0, of 512x64 9.7 -> 5.9; 8 heads of 1000x64 16.3 -> 8.1.
+// ---------------------------------------------------------------------------
+template <typename T, int D, int KS>
+__global__ __launch_bounds__(64 * KS, 2) void attn_fwd_half_keys_kernel(const uint16_t* __restrict__ Q,
+                                                                        const uint16_t* __restrict__ K,
+                                                                        const uint16_t* __restrict__ Vt,
+                                                                        float* __restrict__ O, int S, int S_pad,
+                                                                        int causal, float scale) {
+  constexpr int KT = 64;
+  constexpr int KCH = D / 8;            // 16-byte chunks per K row
+  constexpr int K_RPI = 64 / KCH;       // K rows per 1 KB load instruction
+  constexpr int TILE = KT * D;          // elements of a K (or V^T) tile
+  constexpr int NL = TILE * 2 / 1024;   // load instructions per tile
+  constexpr int OS = D + 4;             // row stride of a parked O
+  static_assert(32 * OS + 64 <= TILE, "a wave's state fits in its tiles");
+  static_assert(KS * 2 * TILE * 2 <= 160 * 1024, "LDS");
+  // KS 2 TILE elements, sized by the launch: with a static size the compiler
+  // sees one workgroup per CU and spreads the accumulators over AGPRs (112
+  // moves a tile at D = 128).
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q0 = (static_cast<int>(gridDim.y) - 1 - static_cast<int>(blockIdx.y)) * 32;  // heaviest (causal) first
+  const int bh = blockIdx.x;
+  const size_t hoff = static_cast<size_t>(bh) * S_pad * D;
+  const uint16_t* Kh = K + hoff;
+  const uint16_t* Vh = Vt + hoff;
+  // The swizzles repeat every 16 rows: PK (of K) or 2 (of V^T) instructions.
+  constexpr int PK = 16 / K_RPI;
+  uint32_t k_off[PK];
+  uint32_t v_off[2];
+#pragma unroll
+  for (int i = 0; i < PK; ++i) {
+    const int kr = K_RPI * i + lane / KCH;
+    const int kswz = KCH == 16 ? (kr & 15) : ((kr >> 1) & 7);
+    k_off[i] = static_cast<uint32_t>(kr * D + ((lane % KCH) ^ kswz) * 8) * 2u;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int vr = 8 * i + (lane >> 3);
+    v_off[i] = static_cast<uint32_t>(vr * S_pad + ((lane & 7) ^ ((vr >> 1) & 7)) * 8) * 2u;
+  }
+  uint16_t* ks = smem + wave * 2 * TILE;
+  uint16_t* vs = ks + TILE;
+  const uint32_t lds0 = lds_addr(smem) + static_cast<uint32_t>(wave) * (4u * TILE);
+  const int kend = causal ? min(S, q0 + 32) : S;
+  const int nt = (kend + KT - 1) / KT;
+  // Refills a buffer that every read issued so far is done with (tiles past
+  // the last: that one again, unused).
+  auto issue_k = [&](int tile) {
+    const uint16_t* base = Kh + static_cast<size_t>(min(tile, nt - 1)) * KT * D;
+    asm volatile("" ::: "memory");
+    wait_lgkmcnt<0>();
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      load_lds16_sbase(k_off[i % PK], base + (i / PK) * 16 * D, lds0 + 1024u * i);
+    }
+  };
+  auto issue_v = [&](int tile) {
+    const uint16_t* base = Vh + min(tile, nt - 1) * KT;
+    asm volatile("" ::: "memory");
+    wait_lgkmcnt<0>();
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      load_lds16_sbase(v_off[i % 2], base + static_cast<size_t>(i / 2) * 16 * S_pad, lds0 + 2u * TILE + 1024u * i);
+    }
+  };
+
+  HalfAttnWave<T, D> w;
+  w.init(Q + hoff + static_cast<size_t>(q0 + (lane & 31)) * D, q0, S, causal, scale, lane);
+  floatx16 s_a[2];
+  floatx16 s_b[2];
+  if (wave < nt) {
+    issue_k(wave);
+    wait_vmcnt<0>();
+    asm volatile("" ::: "memory");
+    w.qk(ks, s_a);
+    issue_k(wave + KS);
+    issue_v(wave);
+    auto tile = [&](int j, floatx16 (&s_cur)[2], floatx16 (&s_nxt)[2]) {
+      u32x4 pb[4];
+      wait_vmcnt<NL>();  // K(j + KS) is here; V^T(j) may be on its way
+      asm volatile("" ::: "memory");
+      w.probabilities(j, ks, s_cur, s_nxt, pb);
+      issue_k(j + 2 * KS);
+      wait_vmcnt<NL>();  // V^T(j) is here
+      asm volatile("" ::: "memory");
+      w.values(vs, pb);
+      issue_v(j + KS);
+    };
+    for (int j = wave; j < nt; j += 2 * KS) {
+      tile(j, s_a, s_b);
+      if (j + KS < nt) {
+        tile(j + KS, s_b, s_a);
+      }
+    }
+    wait_vmcnt<0>();  // no copy may still be writing LDS
+    asm volatile("" ::: "memory");
+  }
+
+  // Each wave parks O as [query][d], its reference and row sum over its own
+  // tiles; a query that saw no valid key in a wave weighs nothing there.
+  float* mine = reinterpret_cast<float*>(ks);
+  const float l_tot = w.l_run + __shfl_xor(w.l_run, 32);
+#pragma unroll
+  for (int t = 0; t < w.DT; ++t) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      *reinterpret_cast<float4*>(mine + w.lrow * OS + t * 32 + 8 * g + 4 * w.half) =
+          make_float4(w.o[t][4 * g], w.o[t][4 * g + 1], w.o[t][4 * g + 2], w.o[t][4 * g + 3]);
+    }
+  }
+  if (w.half == 0) {
+    mine[32 * OS + w.lrow] = w.started ? w.m_run : kMaskValue;
+    mine[32 * OS + 32 + w.lrow] = l_tot;
+  }
+  __syncthreads();
+  const float* park = reinterpret_cast<const float*>(smem);
+  for (int u = threadIdx.x; u < 32 * (D / 4); u += 64 * KS) {
+    const int q = u / (D / 4);
+    const int d = (u - q * (D / 4)) * 4;
+    float m_all = kMaskValue;
+#pragma unroll
+    for (int y = 0; y < KS; ++y) {
+      m_all = fmaxf(m_all, park[y * TILE + 32 * OS + q]);
+    }
+    float l_all = 0.0f;
+    float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int y = 0; y < KS; ++y) {
+      const float f = fast_exp2(park[y * TILE + 32 * OS + q] - m_all);
+      const float4 v = *reinterpret_cast<const float4*>(park + y * TILE + q * OS + d);
+      l_all += f * park[y * TILE + 32 * OS + 32 + q];
+      acc.x += f * v.x;
+      acc.y += f * v.y;
+      acc.z += f * v.z;
+      acc.w += f * v.w;
+    }
+    const float inv = 1.0f / l_all;
+    if (q0 + q < S) {
+      *reinterpret_cast<float4*>(O + (static_cast<size_t>(bh) * S + q0 + q) * D + d) =
+          make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    }
+  }
+}
+
+template <typename T, int D, int KS>
+static hipError_t launch_half_keys(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out, int bh, int S,
+                                   int S_pad, int causal, float scale, hipStream_t stream) {
+  constexpr int kLds = KS * 2 * 64 * D * 2;
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(attn_fwd_half_keys_kernel<T, D, KS>), hipFuncAttributeMaxDynamicSharedMemorySize,
+      kLds);
+  if (attr != hipSuccess) {
+    return attr;
+  }
+  hipLaunchKernelGGL((attn_fwd_half_keys_kernel<T, D, KS>), dim3(bh, (S + 31) / 32), dim3(64 * KS), kLds, stream, q,
+                     k, vt, out, S, S_pad, causal, scale);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -2440,34 +2624,67 @@ hipError_t vitQkvAttention(const uint16_t* tokens, const uint16_t* Wqkv_t, uint1
   return hipGetLastError();
 }
 
+// How many waves share a query block's keys (attn_fwd_half_keys_kernel), or 1
+// for attn_fwd_half_kernel.  With W 32-query blocks in all, four waves a block
+// win while the blocks fit the chip at once (one per CU at D = 128, two at
+// D = 64 run slower, so up to 1.5 per CU), two waves until the K and V^T tiles
+// that every 32 queries load again cost more than the shorter chain saves;
+// causal blocks average half of the tiles and gain for longer.  Measured at the
+// lines (us: whole blocks of 128 / four / two waves; b x h x S x D):
+//   D 64   1x12x700 12.7/9.3/10.9  4x12x196 7.4/7.1/7.1  1x12x1400 21.2/19.8/18.2
+//          4x12x350 9.3/12.0/9.2   2x12x1400 29.2/30.3/29.9
+//   causal 1x12x1400 21.4/11.8/13.8  4x12x350 9.4/9.4/8.2  2x12x1400 22.4/20.6/18.9
+//          4x16x700 15.0/20.3/16.6
+//   D 128  1x4x1400 29.1/14.6/18.2  2x12x350 12.8/16.5/12.4  1x4x2800 52.1/37.8/40.4
+//          4x16x196 11.0/14.7/10.8  2x12x700 18.8/27.8/25.4
+//   causal 1x12x700 17.4/11.9/13.0  4x16x196 10.6/12.5/9.4  4x12x350 13.3/18.9/15.0
+//          2x12x700 17.9/20.8/15.9  2x12x1400 32.4/42.3/34.9
+static int half_key_shares(int bh, int S, int D, bool causal, int cus) {
+  const long long blocks = static_cast<long long>(bh) * ((S + 31) / 32);
+  const long long eighths = (blocks * 8 + cus - 1) / cus;  // blocks per CU, in eighths
+  if (D == 64) {
+    return eighths <= 12 ? 4 : eighths <= (causal ? 34 : 17) ? 2 : 1;
+  }
+  return eighths <= 8 ? 4 : eighths <= (!causal ? 12 : S < 512 ? 14 : 17) ? 2 : 1;
+}
+
 hipError_t attentionHalf(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out_f32,
                          uint16_t* out_heads_concat, int heads, int bh, int S, int S_pad, int D, bool causal, Half t,
-                         hipStream_t stream) {
+                         int cus, hipStream_t stream) {
   // The K / V^T copies use 32-bit byte offsets inside one head.
   if (S <= 0 || bh <= 0 || S_pad % 128 != 0 || S_pad < S || (D != 64 && D != 128) ||
       static_cast<long long>(S_pad) * D * 2 >= (1LL << 31)) {
     return hipErrorInvalidValue;
   }
   const float scale = 1.0f / sqrtf(static_cast<float>(D));
-  const dim3 grid(bh, S_pad / 128);
   const int cz = causal ? 1 : 0;
+#define LC_ATTN_HALF(KERNEL, GRID_Y, THREADS)                                                                     \
+  hipLaunchKernelGGL(KERNEL, dim3(bh, GRID_Y), dim3(THREADS), 0, stream, q, k, vt, out_f32, out_heads_concat, heads, \
+                     S, S_pad, cz, scale)
+  // The heads-concatenated output is the ViT block's, whose fused kernel
+  // computes what attn_fwd_half_kernel does, bit for bit.
+  if (const int ks = half_key_shares(bh, S, D, causal, cus); ks > 1 && out_heads_concat == nullptr) {
+#define LC_HALF_KEYS(T_, D_)                                                                       \
+  (ks == 4 ? launch_half_keys<T_, D_, 4>(q, k, vt, out_f32, bh, S, S_pad, cz, scale, stream) \
+           : launch_half_keys<T_, D_, 2>(q, k, vt, out_f32, bh, S, S_pad, cz, scale, stream))
+    if (t == Half::kBF16) {
+      return D == 64 ? LC_HALF_KEYS(BF16, 64) : LC_HALF_KEYS(BF16, 128);
+    }
+    return D == 64 ? LC_HALF_KEYS(F16, 64) : LC_HALF_KEYS(F16, 128);
+#undef LC_HALF_KEYS
+  }
   if (t == Half::kBF16) {
     if (D == 64) {
-      hipLaunchKernelGGL((attn_fwd_half_kernel<BF16, 64>), grid, dim3(256), 0, stream, q, k, vt, out_f32,
-                         out_heads_concat, heads, S, S_pad, cz, scale);
+      LC_ATTN_HALF((attn_fwd_half_kernel<BF16, 64>), S_pad / 128, 256);
     } else {
-      hipLaunchKernelGGL((attn_fwd_half_kernel<BF16, 128>), grid, dim3(256), 0, stream, q, k, vt, out_f32,
-                         out_heads_concat, heads, S, S_pad, cz, scale);
+      LC_ATTN_HALF((attn_fwd_half_kernel<BF16, 128>), S_pad / 128, 256);
     }
+  } else if (D == 64) {
+    LC_ATTN_HALF((attn_fwd_half_kernel<F16, 64>), S_pad / 128, 256);
   } else {
-    if (D == 64) {
-      hipLaunchKernelGGL((attn_fwd_half_kernel<F16, 64>), grid, dim3(256), 0, stream, q, k, vt, out_f32,
-                         out_heads_concat, heads, S, S_pad, cz, scale);
-    } else {
-      hipLaunchKernelGGL((attn_fwd_half_kernel<F16, 128>), grid, dim3(256), 0, stream, q, k, vt, out_f32,
-                         out_heads_concat, heads, S, S_pad, cz, scale);
-    }
+    LC_ATTN_HALF((attn_fwd_half_kernel<F16, 128>), S_pad / 128, 256);
   }
+#undef LC_ATTN_HALF
   return hipGetLastError();
 }
 

@@ -10,14 +10,12 @@
 //    as consecutive S*D slices of the flat NCHW output, repeated when short
 //    (QkvPackRepeat :709-729), then single-head attention.  Every stage stays
 //    in device memory (the reference round-trips through host vectors).
-//  * The ViT block chains three kernels on one stream: the patch-embed conv
+//  * The ViT block chains four kernels on one stream: the patch-embed conv
 //    (+ReLU) as a row-major GEMM on the input stored as patch rows (the
 //    stride-P conv's im2col is a permutation of the image, applied once at
-//    upload) writing tokens [B*T, E]; the QKV projection fused with attention
-//    per (image, head), Q/K/V^T kept in LDS, writing heads concatenated
-//    [B*T, E]; the output projection.  CJ_HIP_VIT_PATCHIFY=0 and
-//    CJ_HIP_VIT_FUSED=0 select the implicit-im2col GEMM and the separate QKV
-//    GEMM (head-major Q/K, transposed V) + attention kernels.
+//    upload) writing tokens [B*T, E]; the QKV projection (head-major Q / K,
+//    transposed V); attention, writing heads concatenated [B*T, E]; the output
+//    projection.  CJ_HIP_VIT_PATCHIFY=0 selects the implicit-im2col GEMM.
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
@@ -314,13 +312,6 @@ bool vitPatchifyEnabled() {
   return env == nullptr || std::string(env) != "0";
 }
 
-// The fused QKV + attention kernel is the default where it fits;
-// CJ_HIP_VIT_FUSED=0 selects the separate QKV GEMM and attention kernels.
-bool vitFusedEnabled() {
-  const char* env = getenv("CJ_HIP_VIT_FUSED");
-  return env == nullptr || std::string(env) != "0";
-}
-
 Status vitForwardDevice(HipContext* ctx, lcVitBlockSession* s) {
   const auto& c = s->cfg;
   const kern::Half ht = halfOf(c.compute_dtype);
@@ -329,10 +320,11 @@ Status vitForwardDevice(HipContext* ctx, lcVitBlockSession* s) {
   const int H = static_cast<int>(c.heads);
   const int T = static_cast<int>(s->T);
   const int M = static_cast<int>(s->M);
+  const int cus = ctx->props.multiProcessorCount;
   traceOpDispatch(TraceOp::kConv2dNchw, Device::kHIP, Device::kHIP, false, s->M * c.embed * s->K);
   hipError_t e = s->patchify
                      ? kern::patchTokensGemm(s->x16.as<uint16_t>(), s->wconv16.as<uint16_t>(), s->tokens16.as<uint16_t>(),
-                                             M, static_cast<int>(s->K), E, ht, ctx->stream)
+                                             M, static_cast<int>(s->K), E, ht, cus, ctx->stream)
                      : kern::patchEmbedGemm(s->x16.as<uint16_t>(), s->wconv16.as<uint16_t>(),
                                             s->tokens16.as<uint16_t>(), B, static_cast<int>(c.in_channels),
                                             static_cast<int>(c.image_h), static_cast<int>(c.image_w),
@@ -341,36 +333,22 @@ Status vitForwardDevice(HipContext* ctx, lcVitBlockSession* s) {
     return failHip(e, "vit patch-embed launch");
   }
   traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, s->M * c.embed * 3 * c.embed);
-  if (vitFusedEnabled() && kern::vitQkvAttentionFits(T, E, H)) {
-    // QKV projection and attention in one launch per (image, head): Q, K and
-    // V^T stay in LDS.
-    traceOpDispatch(TraceOp::kAttentionForward, Device::kHIP, Device::kHIP, false, s->T * s->T * s->Dh);
-    e = kern::vitQkvAttention(s->tokens16.as<uint16_t>(), s->wqkv_t16.as<uint16_t>(), s->attn16.as<uint16_t>(), B, T,
-                              E, H, ht, ctx->stream);
-    if (e != hipSuccess) {
-      return failHip(e, "vit qkv + attention launch");
-    }
-    traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, s->M * c.embed * c.embed);
-    e = kern::outProjectGemm(s->attn16.as<uint16_t>(), s->wo_t16.as<uint16_t>(), s->out.as<float>(), M, E, ht,
-                             ctx->stream);
-    return e == hipSuccess ? Status::kSuccess : failHip(e, "vit out-projection launch");
-  }
   e = kern::qkvProjectGemm(s->tokens16.as<uint16_t>(), s->wqkv_t16.as<uint16_t>(), s->q16.as<uint16_t>(),
                            s->k16.as<uint16_t>(), s->vt16.as<uint16_t>(), B, T, E, H, static_cast<int>(s->S_pad), ht,
-                           ctx->stream);
+                           cus, ctx->stream);
   if (e != hipSuccess) {
     return failHip(e, "vit qkv launch");
   }
   traceOpDispatch(TraceOp::kAttentionForward, Device::kHIP, Device::kHIP, false, s->T * s->T * s->Dh);
   e = kern::attentionHalf(s->q16.as<uint16_t>(), s->k16.as<uint16_t>(), s->vt16.as<uint16_t>(), nullptr,
                           s->attn16.as<uint16_t>(), H, B * H, T, static_cast<int>(s->S_pad), static_cast<int>(s->Dh),
-                          false, ht, ctx->props.multiProcessorCount, ctx->stream);
+                          false, ht, cus, ctx->stream);
   if (e != hipSuccess) {
     return failHip(e, "vit attention launch");
   }
   traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, s->M * c.embed * c.embed);
   e = kern::outProjectGemm(s->attn16.as<uint16_t>(), s->wo_t16.as<uint16_t>(), s->out.as<float>(), M, E, ht,
-                           ctx->stream);
+                           cus, ctx->stream);
   return e == hipSuccess ? Status::kSuccess : failHip(e, "vit out-projection launch");
 }
 

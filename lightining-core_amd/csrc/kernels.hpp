@@ -295,6 +295,12 @@ inline bool isR4(GemmHalfVariant v) { return v >= GemmHalfVariant::kR128; }
 GemmHalfVariant gemmHalfR4Choose(int M, int N, int K, int cus);
 hipError_t gemmHalfR4(const uint16_t* A, const uint16_t* Bt, float* C, int M, int N, int K, int lda, int ldb, int ldc,
                       Half t, GemmHalfVariant variant, hipStream_t stream);
+// relu(C) in 16 bits (N % 4 == 0, ldc % 4 == 0), and the QKV projection of
+// qkvProjectGemm, on the same kernels.  Both operands padded as above.
+hipError_t gemmHalfR4Relu(const uint16_t* A, const uint16_t* Bt, uint16_t* C, int M, int N, int K, int lda, int ldb,
+                          int ldc, Half t, int cus, hipStream_t stream);
+hipError_t gemmHalfR4Qkv(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16_t* q, uint16_t* k, uint16_t* vt, int B,
+                         int T_, int E, int H, int S_pad, Half t, int cus, hipStream_t stream);
 // Same GEMM with a 16-bit output (optionally ReLU).
 hipError_t gemmHalfTNHalfOut(const uint16_t* A, const uint16_t* Bt, uint16_t* C, int M, int N, int K, int lda,
                              int ldb, int ldc, int relu, Half t, hipStream_t stream);
@@ -308,16 +314,16 @@ hipError_t patchEmbedGemm(const uint16_t* x, const uint16_t* Wt, uint16_t* token
 // The patch-embed conv as a row-major GEMM on vitPatchify's xp [M][K]:
 // tokens = relu(xp . Wt^T), the same tiles and k order as patchEmbedGemm.
 hipError_t patchTokensGemm(const uint16_t* xp, const uint16_t* Wt, uint16_t* tokens, int M, int K, int E, Half t,
-                           hipStream_t stream);
+                           int cus, hipStream_t stream);
 // QKV projection for the ViT block: qkv = tokens[M, E] . Wqkv_t[3E, E]^T with
 // the epilogue writing head-major Q, K [B*H, S_pad, Dh] and V transposed
 // Vt [B*H, Dh, S_pad] (16-bit), M = B*T, S = T.
 hipError_t qkvProjectGemm(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16_t* q, uint16_t* k, uint16_t* vt,
-                          int B, int T, int E, int H, int S_pad, Half t, hipStream_t stream);
+                          int B, int T, int E, int H, int S_pad, Half t, int cus, hipStream_t stream);
 // ViT output projection: out[M, E] (fp32) = attn[M, E] . Wo_t[E, E]^T (16-bit
 // operands, E % 64 == 0).
 hipError_t outProjectGemm(const uint16_t* attn, const uint16_t* Wo_t, float* out, int M, int E, Half t,
-                          hipStream_t stream);
+                          int cus, hipStream_t stream);
 
 // Flash attention over `bh` problems: Q, K [bh, S_pad, D], Vt [bh, D, S_pad]
 // (16-bit, zero padded to S_pad = roundup(S, 128)), D in {64, 128}.  Output
@@ -326,13 +332,5 @@ hipError_t outProjectGemm(const uint16_t* attn, const uint16_t* Wo_t, float* out
 hipError_t attentionHalf(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out_f32,
                          uint16_t* out_heads_concat, int heads, int bh, int S, int S_pad, int D, bool causal, Half t,
                          int cus, hipStream_t stream);
-
-// ViT: QKV projection of each (image, head) fused with its attention
-// (vit_qkv_attn_kernel); tokens [B*T][E], Wqkv_t [3E][E], output
-// heads-concatenated [B*T][E].  Needs E / H == 64, T <= 224 (the kernel's LDS
-// holds 224 token rows), E % 64 == 0.
-bool vitQkvAttentionFits(int T_, int E, int H);
-hipError_t vitQkvAttention(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16_t* out_heads_concat, int B,
-                           int T_, int E, int H, Half t, hipStream_t stream);
 
 }  // namespace lchip::kern

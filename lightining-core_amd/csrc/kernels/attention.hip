@@ -1309,8 +1309,8 @@ __device__ __forceinline__ u32x4 scale_halves(u32x4 v, float c) {
 
 // Per-wave state and steps of the 16-bit attention: queries q0 .. q0 + 31
 // against 64-key K / V^T tiles in LDS, in the layouts above.  Shared by
-// attn_fwd_half_kernel (tiles streamed through two LDS buffers) and
-// vit_qkv_attn_kernel (every tile resident), so both compute the same values.
+// attn_fwd_half_kernel (a workgroup's waves share each tile) and
+// attn_fwd_half_keys_kernel (every wave has tiles of its own).
 template <typename T, int D>
 struct HalfAttnWave {
   static constexpr int KT = 64;
@@ -1682,8 +1682,9 @@ template <typename T, int D, int KS>
 __global__ __launch_bounds__(64 * KS, 2) void attn_fwd_half_keys_kernel(const uint16_t* __restrict__ Q,
                                                                         const uint16_t* __restrict__ K,
                                                                         const uint16_t* __restrict__ Vt,
-                                                                        float* __restrict__ O, int S, int S_pad,
-                                                                        int causal, float scale) {
+                                                                        float* __restrict__ O,
+                                                                        uint16_t* __restrict__ Ocat, int heads, int S,
+                                                                        int S_pad, int causal, float scale) {
   constexpr int KT = 64;
   constexpr int KCH = D / 8;            // 16-byte chunks per K row
   constexpr int K_RPI = 64 / KCH;       // K rows per 1 KB load instruction
@@ -1816,16 +1817,27 @@ __global__ __launch_bounds__(64 * KS, 2) void attn_fwd_half_keys_kernel(const ui
       acc.w += f * v.w;
     }
     const float inv = 1.0f / l_all;
-    if (q0 + q < S) {
+    if (q0 + q >= S) {
+      continue;
+    }
+    if (Ocat == nullptr) {
       *reinterpret_cast<float4*>(O + (static_cast<size_t>(bh) * S + q0 + q) * D + d) =
           make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    } else {
+      const int b = bh / heads;
+      u32x2 v;
+      v[0] = pack2<T>(acc.x * inv, acc.y * inv);
+      v[1] = pack2<T>(acc.z * inv, acc.w * inv);
+      *reinterpret_cast<u32x2*>(Ocat + (static_cast<size_t>(b) * S + q0 + q) * (heads * D) + (bh - b * heads) * D + d) =
+          v;
     }
   }
 }
 
 template <typename T, int D, int KS>
-static hipError_t launch_half_keys(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out, int bh, int S,
-                                   int S_pad, int causal, float scale, hipStream_t stream) {
+static hipError_t launch_half_keys(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out,
+                                   uint16_t* out_cat, int heads, int bh, int S, int S_pad, int causal, float scale,
+                                   hipStream_t stream) {
   constexpr int kLds = KS * 2 * 64 * D * 2;
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(attn_fwd_half_keys_kernel<T, D, KS>), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1834,388 +1846,8 @@ static hipError_t launch_half_keys(const uint16_t* q, const uint16_t* k, const u
     return attr;
   }
   hipLaunchKernelGGL((attn_fwd_half_keys_kernel<T, D, KS>), dim3(bh, (S + 31) / 32), dim3(64 * KS), kLds, stream, q,
-                     k, vt, out, S, S_pad, causal, scale);
+                     k, vt, out, out_cat, heads, S, S_pad, causal, scale);
   return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// ViT block: the QKV projection of one (image, head) fused with its
-// attention, so Q, K and V^T never leave LDS.  T <= 224 tokens (nrb =
-// ceil(T/32) <= 7 blocks of 32), head dim 64.  Each (image b, head h) takes
-// nparts = min(2, nrb) workgroups of 8 waves; part p owns a contiguous range
-// of query blocks [qlo, qhi) (at most 4), and every part projects K and V for
-// all tokens (the attention of its queries needs every key), Q only for its
-// own queries.
-//  1. Projection: token rows of image b times the head's 192 rows of W_qkv^T
-//     (Q rows h*64.., K rows E + h*64.., V rows 2E + h*64..), in 64-deep
-//     stages through a ring of three LDS buffers: 224 token rows (rows past T
-//     re-read token T-1, so every value stays finite) and the 192 weight
-//     rows, 128-byte rows with chunk ^ ((row >> 1) & 7), one direct
-//     global -> LDS copy per 8 rows (52 per stage, 6 or 7 per wave).  The
-//     copies of stage s+2 go out during stage s, two after each k-step.
-//     32x32 output blocks ("units") per wave: wave w < nrb takes K and V of
-//     token block w (four units) and, when w is one of this part's query
-//     blocks, Q's first 32 columns; Q's other 32 columns of this part's first
-//     min(3, #query blocks) blocks go to wave 7 and those of the rest stay
-//     with their wave (at T = 196 that is 9 units on every SIMD).  Q and K
-//     units compute W . tokens^T (rows d, columns tokens) and V units
-//     tokens . W^T, so every lane ends up with 4 consecutive elements of one
-//     LDS row below.  v_mfma_f32_32x32x16 in the k order of the QKV GEMM, the
-//     fragments of k-step kk+1 read while kk's MFMAs run.
-//  2. The accumulators go to LDS as 16-bit Q [128][64] (this part's queries),
-//     K tiles [64][64] and V^T tiles [64][64] (keys past the last token block
-//     zero) in attn_fwd_half_kernel's layouts, 8-byte stores.
-//  3. Wave a < #query blocks runs attention for query block qlo + a over
-//     every key tile (HalfAttnWave: attn_fwd_half_kernel's arithmetic) and
-//     stores its rows of the heads-concatenated output.
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(512) void vit_qkv_attn_kernel(const uint16_t* __restrict__ tokens,
-                                                          const uint16_t* __restrict__ Wqkv_t,
-                                                          uint16_t* __restrict__ Ocat, int T_, int E, int H,
-                                                          int nparts, int tb, int th, float scale) {
-  constexpr int D = 64;
-  constexpr int KT = 64;
-  constexpr int TILE = KT * D;            // elements of a K (or V^T) tile
-  constexpr int AR = 224;                 // token rows per stage (padded)
-  constexpr int WR = 3 * D;               // weight rows: Q, K, V of one head
-  constexpr int NB = 3;                   // ring buffers
-  constexpr int STAGE = (AR + WR) * 64;   // elements per projection stage
-  constexpr int NCP = (AR + WR) / 8;      // 1 KB copies per stage (52)
-  constexpr int CPW = (NCP + 7) / 8;      // per wave, at most (7)
-  constexpr int ACP = AR / 8;             // ... of token rows (28)
-  constexpr int QR = 128;                 // Q rows held (4 query blocks)
-  constexpr int SP = 256;                 // keys held by the K / V^T tiles
-  // Phase 2 layout (elements): Q [QR][D] at 0, then the K tiles, then the
-  // V^T tiles.
-  constexpr int KOFF = QR * D;
-  constexpr int VOFF = KOFF + (SP / KT) * TILE;
-  static_assert(VOFF + (SP / KT) * TILE <= NB * STAGE, "phase 2 fits in the projection ring");
-  static_assert(NB * STAGE * 2 <= 160 * 1024, "LDS");
-  __shared__ __attribute__((aligned(16))) uint16_t smem[NB * STAGE];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wave_s = __builtin_amdgcn_readfirstlane(wave);
-  // Workgroup -> (image, head, part).  With tb > 0 the 8 XCDs (workgroup w
-  // runs on XCD w % 8) each take a tb x th block of (image, head) pairs, so
-  // an XCD's L2 fetches the tokens of tb images and the weights of th heads
-  // (the host picks the block that minimises those bytes); else in order.
-  int b;
-  int h;
-  int part;
-  if (tb > 0) {
-    const int x = blockIdx.x & 7;
-    const int l = blockIdx.x >> 3;
-    const int tiles_b = static_cast<int>(gridDim.x) / (H * nparts) / tb;
-    part = l % nparts;
-    const int r = l / nparts;
-    b = (x % tiles_b) * tb + r % tb;
-    h = (x / tiles_b) * th + r / tb;
-  } else {
-    const int q = blockIdx.x / nparts;
-    part = blockIdx.x - q * nparts;
-    b = q / H;
-    h = q - b * H;
-  }
-  const int bh = b * H + h;
-  const uint16_t* tok = tokens + static_cast<size_t>(b) * T_ * E;
-  const int nrb = (T_ + 31) >> 5;
-  const int per = (nrb + nparts - 1) / nparts;
-  const int qlo = part * per;
-  const int nq = min(nrb, qlo + per) - qlo;  // 1..4
-  const int nmove = min(3, nq);              // Q column-block-1 units done by wave 7
-
-  // Copy j of this wave is instruction i = wave + 8j of the stage (i < NCP):
-  // stage rows 8i + lane/8 (token rows for i < ACP, weight rows after),
-  // physical chunk lane % 8 holding logical chunk (lane % 8) ^ ((row >> 1) & 7).
-  // Byte offsets are 32-bit (the host keeps T*E*2 and 3*E*E*2 below 2^31).
-  uint32_t off[CPW];
-  const uint16_t* cbase[CPW];
-#pragma unroll
-  for (int j = 0; j < CPW; ++j) {
-    const int i = wave_s + 8 * j;
-    const int row = 8 * i + (lane >> 3);
-    const int lch = (lane & 7) ^ ((row >> 1) & 7);
-    if (i < ACP) {
-      const int t = min(row, T_ - 1);
-      off[j] = static_cast<uint32_t>(t * E + lch * 8) * 2u;
-      cbase[j] = tok;
-    } else {
-      const int r = min(row - AR, WR - 1);
-      const int wrow = (r >> 6) * E + h * D + (r & 63);
-      off[j] = static_cast<uint32_t>(wrow * E + lch * 8) * 2u;
-      cbase[j] = Wqkv_t;
-    }
-  }
-  const bool full_cpw = wave_s + 8 * (CPW - 1) < NCP;  // CPW copies per stage, else CPW - 1
-  const uint32_t lds0 = lds_addr(smem);
-  // Copies j0 .. j1-1 of stage st into ring slot buf.
-  auto issue = [&](int st, int buf, int j0, int j1) {
-    const int k0 = st * 64;
-#pragma unroll
-    for (int j = 0; j < CPW; ++j) {
-      if (j >= j0 && j < j1 && (j < CPW - 1 || full_cpw)) {
-        load_lds16_sbase(off[j], cbase[j] + k0,
-                         lds0 + 2u * static_cast<uint32_t>(buf * STAGE + (wave_s + 8 * j) * 512));
-      }
-    }
-  };
-
-  const int lrow = lane & 31;
-  const int lhalf = lane >> 5;
-  // Token rows 32w + lrow and weight rows AR + 32cb + lrow share the swizzle
-  // (lrow >> 1) & 7.
-  const int swz = (lrow >> 1) & 7;
-  floatx16 acc[6];
-#pragma unroll
-  for (int u = 0; u < 6; ++u) {
-    acc[u] = zero16();
-  }
-  // Wave roles (uniform): main waves w < nrb hold K0 K1 V0 V1 in acc[0..3],
-  // Q0 in acc[4] when w is a query block of this part, and Q1 in acc[5] when
-  // it is one past the first nmove; wave 7 holds Q1 of query blocks
-  // qlo .. qlo + nmove - 1 in acc[0..nmove-1].
-  const bool main_w = wave_s < nrb;
-  const bool has_q = main_w && wave_s >= qlo && wave_s < qlo + nq;
-  const bool own_q1 = has_q && wave_s - qlo >= nmove;
-  const bool helper = wave_s == 7;
-
-  // The stage loop; compute(sb, cp) runs this wave's 4 k-steps on the stage
-  // at sb and calls cp(kk) after k-step kk's MFMAs, which issues two of the
-  // copies of stage st + 2 (the last k-step the rest): spread over the stage,
-  // the copies do not queue up behind each other at the address unit while
-  // the MFMAs wait.
-  const int nst = E / 64;
-  auto run = [&](auto compute) {
-    issue(0, 0, 0, CPW);
-    if (nst > 1) {
-      issue(1, 1, 0, CPW);
-    }
-    int buf = 0;   // ring slot of stage st
-    int buf2 = 2;  // ring slot of stage st + 2
-    for (int st = 0; st < nst; ++st) {
-      // This wave's copies of stage st have landed (those of st + 1 may still
-      // be in flight), then everyone's have, and everyone is done with stage
-      // st - 1, whose slot takes stage st + 2.
-      if (st + 1 < nst) {
-        if (full_cpw) {
-          wait_vmcnt<CPW>();
-        } else {
-          wait_vmcnt<CPW - 1>();
-        }
-      } else {
-        wait_vmcnt<0>();
-      }
-      stage_barrier();
-      const bool more = st + 2 < nst;
-      auto cp = [&](int kk) {
-        if (more) {
-          issue(st + 2, buf2, 2 * kk, kk == 3 ? CPW : 2 * kk + 2);
-        }
-      };
-      compute(smem + buf * STAGE, cp);
-      buf = buf == NB - 1 ? 0 : buf + 1;
-      buf2 = buf2 == NB - 1 ? 0 : buf2 + 1;
-    }
-  };
-  auto rd_a = [&](const uint16_t* sb, int kk, int rb) {
-    return *reinterpret_cast<const u32x4*>(sb + (rb * 32 + lrow) * 64 + (((2 * kk + lhalf) ^ swz) << 3));
-  };
-  auto rd_w = [&](const uint16_t* sb, int kk, int cb) {
-    return *reinterpret_cast<const u32x4*>(sb + (AR + cb * 32 + lrow) * 64 + (((2 * kk + lhalf) ^ swz) << 3));
-  };
-  // Main waves: NQ = 0, 1 or 2 Q units.  Fragment slots: [0] tokens, [1..4]
-  // K0 K1 V0 V1 weights, [5..] Q0 Q1 weights.
-  auto main_stage = [&](auto nq_c) {
-    constexpr int NQ = decltype(nq_c)::value;
-    constexpr int NF = 5 + NQ;
-    return [&](const uint16_t* sb, auto cp) {
-      u32x4 f[2][NF];
-      auto rd = [&](int kk, u32x4 (&g)[NF]) {
-        g[0] = rd_a(sb, kk, wave_s);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          g[1 + u] = rd_w(sb, kk, 2 + u);
-        }
-#pragma unroll
-        for (int u = 0; u < NQ; ++u) {
-          g[5 + u] = rd_w(sb, kk, u);
-        }
-      };
-      rd(0, f[0]);
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        if (kk < 3) {
-          rd(kk + 1, f[(kk + 1) & 1]);
-        }
-        const u32x4(&g)[NF] = f[kk & 1];
-        acc[0] = mfma32x32x16<T>(g[1], g[0], acc[0]);  // K rows d 0..31
-        acc[1] = mfma32x32x16<T>(g[2], g[0], acc[1]);  // K rows d 32..63
-        acc[2] = mfma32x32x16<T>(g[0], g[3], acc[2]);  // V columns d 0..31
-        acc[3] = mfma32x32x16<T>(g[0], g[4], acc[3]);  // V columns d 32..63
-#pragma unroll
-        for (int u = 0; u < NQ; ++u) {
-          acc[4 + u] = mfma32x32x16<T>(g[5 + u], g[0], acc[4 + u]);  // Q rows d 32u..
-        }
-        cp(kk);
-      }
-    };
-  };
-  // Wave 7: Q1 of NM query blocks.  Fragment slots: [0] Q1 weights, [1..NM]
-  // tokens of blocks qlo ...
-  auto helper_stage = [&](auto nm_c) {
-    constexpr int NM = decltype(nm_c)::value;
-    return [&](const uint16_t* sb, auto cp) {
-      u32x4 f[2][1 + NM];
-      auto rd = [&](int kk, u32x4 (&g)[1 + NM]) {
-        g[0] = rd_w(sb, kk, 1);
-#pragma unroll
-        for (int u = 0; u < NM; ++u) {
-          g[1 + u] = rd_a(sb, kk, qlo + u);
-        }
-      };
-      rd(0, f[0]);
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        if (kk < 3) {
-          rd(kk + 1, f[(kk + 1) & 1]);
-        }
-        const u32x4(&g)[1 + NM] = f[kk & 1];
-#pragma unroll
-        for (int u = 0; u < NM; ++u) {
-          acc[u] = mfma32x32x16<T>(g[0], g[1 + u], acc[u]);
-        }
-        cp(kk);
-      }
-    };
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I1 = std::integral_constant<int, 1>;
-  using I2 = std::integral_constant<int, 2>;
-  using I3 = std::integral_constant<int, 3>;
-  if (main_w) {
-    if (!has_q) {
-      run(main_stage(I0{}));
-    } else if (!own_q1) {
-      run(main_stage(I1{}));
-    } else {
-      run(main_stage(I2{}));
-    }
-  } else if (helper) {
-    if (nmove == 1) {
-      run(helper_stage(I1{}));
-    } else if (nmove == 2) {
-      run(helper_stage(I2{}));
-    } else {
-      run(helper_stage(I3{}));
-    }
-  } else {
-    run([](const uint16_t*, auto cp) {
-      cp(0);
-      cp(1);
-      cp(2);
-      cp(3);
-    });
-  }
-  __syncthreads();  // every wave is done with the projection buffers
-
-  // Q, K and V^T to LDS.  In a W . tokens^T unit, register 4g + i of lane l
-  // holds d = 32cb + 8g + 4(l/32) + i of token 32rb + l%32; in a tokens . W^T
-  // unit, token 32rb + 8g + 4(l/32) + i and d = 32cb + l%32.
-  uint16_t* Qs = smem;
-  uint16_t* Ks = smem + KOFF;
-  uint16_t* Vs = smem + VOFF;
-  auto store_q = [&](const floatx16& a, int rb, int cb) {
-    const int t = rb * 32 + lrow;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d0 = cb * 32 + 8 * g + 4 * lhalf;
-      u32x2 v;
-      v[0] = pack2<T>(a[4 * g], a[4 * g + 1]);
-      v[1] = pack2<T>(a[4 * g + 2], a[4 * g + 3]);
-      *reinterpret_cast<u32x2*>(Qs + (t - qlo * 32) * D + d0) = v;
-    }
-  };
-  if (main_w) {
-    const int t = wave_s * 32 + lrow;
-    const int r = t & (KT - 1);
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int d0 = cb * 32 + 8 * g + 4 * lhalf;
-        u32x2 v;
-        v[0] = pack2<T>(acc[cb][4 * g], acc[cb][4 * g + 1]);
-        v[1] = pack2<T>(acc[cb][4 * g + 2], acc[cb][4 * g + 3]);
-        *reinterpret_cast<u32x2*>(Ks + (t / KT) * TILE + r * D + (((d0 >> 3) ^ ((r >> 1) & 7)) << 3) + (d0 & 7)) = v;
-      }
-    }
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      const int d = cb * 32 + lrow;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int t0 = wave_s * 32 + 8 * g + 4 * lhalf;  // keys t0 .. t0 + 3
-        const int r0 = t0 & (KT - 1);
-        u32x2 v;
-        v[0] = pack2<T>(acc[2 + cb][4 * g], acc[2 + cb][4 * g + 1]);
-        v[1] = pack2<T>(acc[2 + cb][4 * g + 2], acc[2 + cb][4 * g + 3]);
-        uint16_t* vdst = Vs + (t0 / KT) * TILE + d * KT + (((r0 >> 3) ^ ((d >> 1) & 7)) << 3) + (r0 & 7);
-        *reinterpret_cast<u32x2*>(vdst) = v;
-      }
-    }
-    if (has_q) {
-      store_q(acc[4], wave_s, 0);
-      if (own_q1) {
-        store_q(acc[5], wave_s, 1);
-      }
-    }
-  } else if (helper) {
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      if (u < nmove) {
-        store_q(acc[u], qlo + u, 1);
-      }
-    }
-    if (nrb & 1) {
-      // Keys 32 nrb .. 32 nrb + 31 (the second half of the last key tile):
-      // zeros (masked keys, whose V rows must stay finite).  K rows 32..63 of
-      // that tile are contiguous; V^T rows d hold them in logical chunks 4..7.
-      const int tl = nrb >> 1;
-      const u32x4 z = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int c = lane + 64 * q;  // 0..255
-        *reinterpret_cast<u32x4*>(Ks + tl * TILE + 32 * D + 8 * c) = z;
-        const int d = c >> 2;
-        const int lc = 4 + (c & 3);
-        *reinterpret_cast<u32x4*>(Vs + tl * TILE + d * KT + ((lc ^ ((d >> 1) & 7)) << 3)) = z;
-      }
-    }
-  }
-  __syncthreads();
-
-  if (wave < nq) {
-    const int q0 = (qlo + wave) * 32;
-    HalfAttnWave<T, D> w;
-    w.init(Qs + (wave * 32 + lrow) * D, q0, T_, 0, scale, lane);
-    const int nt = (T_ + KT - 1) / KT;
-    floatx16 s_a[2];
-    floatx16 s_b[2];
-    w.qk(Ks, s_a);
-    // Every tile is resident: no loads or barriers between tiles.  Past the
-    // last tile the next tile's scores come from the last K tile and go
-    // unused.
-    for (int j = 0; j < nt; j += 2) {
-      w.step(j, Ks + min(j + 1, nt - 1) * TILE, Vs + j * TILE, s_a, s_b);
-      if (j + 1 < nt) {
-        w.step(j + 1, Ks + min(j + 2, nt - 1) * TILE, Vs + (j + 1) * TILE, s_b, s_a);
-      }
-    }
-    w.store(nullptr, Ocat, bh, H);
-  }
 }
 
 }  // namespace lchip::k
@@ -2577,53 +2209,6 @@ hipError_t mseLossF32(const float* out, const float* target, size_t n, float nor
   return hipGetLastError();
 }
 
-bool vitQkvAttentionFits(int T_, int E, int H) {
-  return H > 0 && E % H == 0 && E / H == 64 && T_ > 0 && T_ <= 224 && E % 64 == 0 &&
-         static_cast<long long>(T_) * E * 2 < (1LL << 31) && 3LL * E * E * 2 < (1LL << 31);
-}
-
-hipError_t vitQkvAttention(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16_t* out_heads_concat, int B,
-                           int T_, int E, int H, Half t, hipStream_t stream) {
-  if (B <= 0 || !vitQkvAttentionFits(T_, E, H)) {
-    return hipErrorInvalidValue;
-  }
-  const float scale = 1.0f / sqrtf(64.0f);
-  // Two workgroups per (image, head) once there are two query blocks.
-  const int nparts = T_ > 32 ? 2 : 1;
-  const dim3 grid(B * H * nparts);
-  // XCD blocks: tb images x th heads per XCD, tb | B, th | H, 8 blocks;
-  // per XCD the L2 misses the tokens of tb images (T rows) and the weights
-  // of th heads (192 rows), so minimise tb * T + th * 192.
-  int tb = 0;
-  int th = 0;
-  if ((B * H) % 8 == 0) {
-    long long best = -1;
-    for (int cb = 1; cb <= B; ++cb) {
-      if (B % cb != 0 || (B * H / 8) % cb != 0) {
-        continue;
-      }
-      const int ch = B * H / 8 / cb;
-      if (H % ch != 0) {
-        continue;
-      }
-      const long long cost = static_cast<long long>(cb) * T_ + 192LL * ch;
-      if (best < 0 || cost < best) {
-        best = cost;
-        tb = cb;
-        th = ch;
-      }
-    }
-  }
-  if (t == Half::kBF16) {
-    hipLaunchKernelGGL((vit_qkv_attn_kernel<BF16>), grid, dim3(512), 0, stream, tokens, Wqkv_t, out_heads_concat,
-                       T_, E, H, nparts, tb, th, scale);
-  } else {
-    hipLaunchKernelGGL((vit_qkv_attn_kernel<F16>), grid, dim3(512), 0, stream, tokens, Wqkv_t, out_heads_concat, T_,
-                       E, H, nparts, tb, th, scale);
-  }
-  return hipGetLastError();
-}
-
 // How many waves share a query block's keys (attn_fwd_half_keys_kernel), or 1
 // for attn_fwd_half_kernel.  With W 32-query blocks in all, four waves a block
 // win while the blocks fit the chip at once (one per CU at D = 128, two at
@@ -2661,12 +2246,10 @@ hipError_t attentionHalf(const uint16_t* q, const uint16_t* k, const uint16_t* v
 #define LC_ATTN_HALF(KERNEL, GRID_Y, THREADS)                                                                     \
   hipLaunchKernelGGL(KERNEL, dim3(bh, GRID_Y), dim3(THREADS), 0, stream, q, k, vt, out_f32, out_heads_concat, heads, \
                      S, S_pad, cz, scale)
-  // The heads-concatenated output is the ViT block's, whose fused kernel
-  // computes what attn_fwd_half_kernel does, bit for bit.
-  if (const int ks = half_key_shares(bh, S, D, causal, cus); ks > 1 && out_heads_concat == nullptr) {
-#define LC_HALF_KEYS(T_, D_)                                                                       \
-  (ks == 4 ? launch_half_keys<T_, D_, 4>(q, k, vt, out_f32, bh, S, S_pad, cz, scale, stream) \
-           : launch_half_keys<T_, D_, 2>(q, k, vt, out_f32, bh, S, S_pad, cz, scale, stream))
+  if (const int ks = half_key_shares(bh, S, D, causal, cus); ks > 1) {
+#define LC_HALF_KEYS(T_, D_)                                                                                           \
+  (ks == 4 ? launch_half_keys<T_, D_, 4>(q, k, vt, out_f32, out_heads_concat, heads, bh, S, S_pad, cz, scale, stream) \
+           : launch_half_keys<T_, D_, 2>(q, k, vt, out_f32, out_heads_concat, heads, bh, S, S_pad, cz, scale, stream))
     if (t == Half::kBF16) {
       return D == 64 ? LC_HALF_KEYS(BF16, 64) : LC_HALF_KEYS(BF16, 128);
     }

@@ -300,54 +300,6 @@ struct EpiQKV {
       vt[(head * Dh + d) * S_pad + t] = bits;
     }
   }
-  // A whole 32x32 accumulator of one lane: column n (one head and d for the
-  // lane), rows mbase + 8g + 4*(lane/32) + i, i < 4, for g < 4.  Each group of
-  // 4 rows lies in one image when T_ % 4 == 0 (the caller checks), so its
-  // token index comes from one division and its 4 V^T values are one 8-byte
-  // store; Q and K rows stay 2-byte stores, 32 lanes to 64 contiguous bytes.
-  static constexpr bool kAccStore = true;
-  __device__ __forceinline__ void store_acc(int mbase, int n, const floatx16& acc, int lane, int M, int N) const {
-    if (n >= N) {
-      return;
-    }
-    const int which = n / E;
-    const int r = n - which * E;
-    const int h = r / Dh;
-    const int d = r - h * Dh;
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int m0 = mbase + 8 * g + 4 * (lane >> 5);
-      if (m0 >= M) {
-        continue;
-      }
-      const int b = m0 / T_;
-      const int t0 = m0 - b * T_;
-      const size_t head = static_cast<size_t>(b) * H + h;
-      if (which == 2) {
-        u32x2 w;
-        w[0] = pack2<T>(acc[4 * g], acc[4 * g + 1]);
-        w[1] = pack2<T>(acc[4 * g + 2], acc[4 * g + 3]);
-        *reinterpret_cast<u32x2*>(vt + (head * Dh + d) * S_pad + t0) = w;
-      } else {
-        uint16_t* dst = (which == 0 ? q : k) + (head * S_pad + t0) * Dh + d;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          dst[i * Dh] = to_half_bits<T>(acc[4 * g + i]);
-        }
-      }
-    }
-  }
-};
-
-// Whether an epilogue stores whole accumulators (store_acc) instead of
-// single elements.
-template <typename E, typename = void>
-struct AccStore {
-  static constexpr bool value = false;
-};
-template <typename E>
-struct AccStore<E, decltype(void(E::kAccStore))> {
-  static constexpr bool value = E::kAccStore;
 };
 
 template <typename T, int BM, int BN, int BK, int WM, int WN, int STORE_AT, typename LoadA, typename Epi>
@@ -1673,7 +1625,8 @@ __global__ __launch_bounds__(256) void gemm_half_tn_w4h_kernel(const uint16_t* _
 }
 
 // ---------------------------------------------------------------------------
-// Ring-pipelined 16-bit TN GEMM for short K (the ViT block's GEMMs, K = 768).
+// Ring-pipelined 16-bit TN GEMM for short K (the ViT block's implicit-im2col
+// patch GEMM, K = 768).
 //
 // With K = 768 a tile has 12 stages of BK = 64 and each stage holds only a
 // few MFMAs per wave, so a loop that prefetches one stage ahead pays a global
@@ -1682,22 +1635,9 @@ __global__ __launch_bounds__(256) void gemm_half_tn_w4h_kernel(const uint16_t* _
 // Copies are scalar-base global -> LDS (load_lds16_sbase) with the 128-byte
 // row swizzle of gemm_half_tn_lds_kernel; per-lane offsets are fixed for the
 // tile and rows past M (or N) are clamped to the last row (read, computed,
-// never stored).  The A source is a policy: row-major, or the implicit
-// im2col of a patch-embedding convolution.
+// never stored).  The A source is a policy: the implicit im2col of a
+// patch-embedding convolution.
 // ---------------------------------------------------------------------------
-
-// Row-major A [M, lda]: stage base = tile row bm, column k0.
-struct RingRowMajor {
-  const uint16_t* A;
-  int lda;
-  __device__ __forceinline__ const uint16_t* stage_base(int bm, int k0) const {
-    return A + static_cast<size_t>(bm) * lda + k0;
-  }
-  // Byte offset of (row, k0 + kk) from stage_base(bm, k0), row in [bm, M).
-  __device__ __forceinline__ uint32_t lane_offset(int bm, int row, int kk) const {
-    return static_cast<uint32_t>((row - bm) * lda + kk) * 2u;
-  }
-};
 
 // Implicit im2col of a patch-embedding convolution (kernel = stride = P, no
 // padding) over x [B, C, H, W]: row = b*T + ty*gw + tx, k = (c*P + ky)*P + kx.
@@ -1896,15 +1836,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_half_ring_kernel(ASrc asrc, 
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       const int n = bn + wn + j * 32 + lrow;
-      if constexpr (AccStore<Epi>::value) {
-        epi.store_acc(bm + wm + i * 32, n, acc[i][j], lane, M, N);
-      } else {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = bm + wm + i * 32 + acc_row(r, lane);
-          if (m < M && n < N) {
-            epi(m, n, acc[i][j][r]);
-          }
+      for (int r = 0; r < 16; ++r) {
+        const int m = bm + wm + i * 32 + acc_row(r, lane);
+        if (m < M && n < N) {
+          epi(m, n, acc[i][j][r]);
         }
       }
     }
@@ -2379,7 +2315,8 @@ static hipError_t launch_gemm_ring(ASrc asrc, const uint16_t* Bt, int M, int N, 
   return hipGetLastError();
 }
 
-// The ring kernel serves the ViT GEMMs unless CJ_HIP_VIT_RING is 0 (A/B runs).
+// The ViT GEMMs run on ring-pipelined kernels unless CJ_HIP_VIT_RING is 0 (A/B
+// runs).
 inline bool vit_ring_enabled() {
   const char* env = getenv("CJ_HIP_VIT_RING");
   return env == nullptr || std::string(env) != "0";
@@ -2390,6 +2327,10 @@ inline bool vit_ring_bk128(long long K) {
   const char* env = getenv("CJ_HIP_VIT_RING_BK");
   return K % 128 == 0 && (env == nullptr || std::string(env) != "64");
 }
+
+// The ViT GEMMs with row-major operands take the tiles of gemm_half_tn_r4_kernel
+// unless CJ_HIP_VIT_RING is 0.
+inline bool vit_r4(long long ld) { return vit_ring_enabled() && kern::gemmHalfR4Fits(ld, ld); }
 
 // Its copies use 32-bit byte offsets from a stage base and 16-byte alignment.
 inline bool ring_fits(long long rows, long long ld) { return rows * ld * 2 < (1LL << 31) && ld % 8 == 0; }
@@ -2650,22 +2591,12 @@ hipError_t patchEmbedGemm(const uint16_t* x, const uint16_t* Wt, uint16_t* token
 }
 
 hipError_t patchTokensGemm(const uint16_t* xp, const uint16_t* Wt, uint16_t* tokens, int M, int K, int E, Half t,
-                           hipStream_t stream) {
+                           int cus, hipStream_t stream) {
   if (K % kHBK != 0) {
     return hipErrorInvalidValue;
   }
-  if (vit_ring_enabled() && ring_fits(128, K)) {
-    const RingRowMajor ra{xp, K};
-    if (vit_ring_bk128(K)) {
-      if (t == Half::kBF16) {
-        return launch_gemm_ring<BF16, 128, 64, 4, 2, 3, 128>(ra, Wt, M, E, K, K, EpiHalf<BF16>{tokens, E, 1}, stream);
-      }
-      return launch_gemm_ring<F16, 128, 64, 4, 2, 3, 128>(ra, Wt, M, E, K, K, EpiHalf<F16>{tokens, E, 1}, stream);
-    }
-    if (t == Half::kBF16) {
-      return launch_gemm_ring<BF16, 128, 64, 4, 2, 4>(ra, Wt, M, E, K, K, EpiHalf<BF16>{tokens, E, 1}, stream);
-    }
-    return launch_gemm_ring<F16, 128, 64, 4, 2, 4>(ra, Wt, M, E, K, K, EpiHalf<F16>{tokens, E, 1}, stream);
+  if (vit_r4(K)) {
+    return gemmHalfR4Relu(xp, Wt, tokens, M, E, K, K, K, E, t, cus, stream);
   }
   const LoadRowMajor la{xp, K};
   if (t == Half::kBF16) {
@@ -2675,26 +2606,14 @@ hipError_t patchTokensGemm(const uint16_t* xp, const uint16_t* Wt, uint16_t* tok
 }
 
 hipError_t qkvProjectGemm(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16_t* q, uint16_t* k, uint16_t* vt,
-                          int B, int T_, int E, int H, int S_pad, Half t, hipStream_t stream) {
+                          int B, int T_, int E, int H, int S_pad, Half t, int cus, hipStream_t stream) {
   const int M = B * T_;
   if (E % kHBK != 0 || E % H != 0) {
     return hipErrorInvalidValue;
   }
   const int Dh = E / H;
-  // The ring kernel's accumulator stores need whole 4-row groups per image.
-  if (vit_ring_enabled() && ring_fits(128, E) && T_ % 4 == 0) {
-    // 128x128 tiles (8 waves): 234 workgroups for the B = 8 block, one per
-    // CU; measured faster than 64x64 tiles (900 workgroups).
-    // 64-deep stages here: a 128-deep stage of this tile is 64 KiB, so only
-    // two fit and one stage is in flight; in the block, where the tokens come
-    // cold from the patch GEMM, that measured 13.2 against 12.9 us.
-    const RingRowMajor ra{tokens, E};
-    if (t == Half::kBF16) {
-      return launch_gemm_ring<BF16, 128, 128, 2, 4, 4>(ra, Wqkv_t, M, 3 * E, E, E,
-                                                       EpiQKV<BF16>{q, k, vt, T_, E, H, Dh, S_pad}, stream);
-    }
-    return launch_gemm_ring<F16, 128, 128, 2, 4, 4>(ra, Wqkv_t, M, 3 * E, E, E,
-                                                    EpiQKV<F16>{q, k, vt, T_, E, H, Dh, S_pad}, stream);
+  if (vit_r4(E)) {
+    return gemmHalfR4Qkv(tokens, Wqkv_t, q, k, vt, B, T_, E, H, S_pad, t, cus, stream);
   }
   const LoadRowMajor la{tokens, E};
   if (t == Half::kBF16) {
@@ -2704,22 +2623,12 @@ hipError_t qkvProjectGemm(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16
 }
 
 hipError_t outProjectGemm(const uint16_t* attn, const uint16_t* Wo_t, float* out, int M, int E, Half t,
-                          hipStream_t stream) {
+                          int cus, hipStream_t stream) {
   if (E % kHBK != 0) {
     return hipErrorInvalidValue;
   }
-  if (vit_ring_enabled() && ring_fits(128, E)) {
-    const RingRowMajor ra{attn, E};
-    if (vit_ring_bk128(E)) {
-      if (t == Half::kBF16) {
-        return launch_gemm_ring<BF16, 128, 64, 4, 2, 3, 128>(ra, Wo_t, M, E, E, E, EpiF32{out, E}, stream);
-      }
-      return launch_gemm_ring<F16, 128, 64, 4, 2, 3, 128>(ra, Wo_t, M, E, E, E, EpiF32{out, E}, stream);
-    }
-    if (t == Half::kBF16) {
-      return launch_gemm_ring<BF16, 128, 64, 4, 2, 4>(ra, Wo_t, M, E, E, E, EpiF32{out, E}, stream);
-    }
-    return launch_gemm_ring<F16, 128, 64, 4, 2, 4>(ra, Wo_t, M, E, E, E, EpiF32{out, E}, stream);
+  if (vit_r4(E)) {
+    return gemmHalfR4(attn, Wo_t, out, M, E, E, E, E, E, t, gemmHalfR4Choose(M, E, E, cus), stream);
   }
   return gemmHalfTN(attn, Wo_t, out, M, E, E, E, E, E, t, GemmHalfVariant::kAuto, stream);
 }

@@ -8,6 +8,90 @@
 
 namespace lchip::k {
 
+// What happens to four consecutive columns n .. n + 3 of row m: row(m) and
+// col(n) hold what the store needs of each, worked out once per lane and block.
+struct StoreF32 {
+  float* C;
+  int ldc;
+  int M, N;
+  int vec4;  // C is 16-byte aligned and ldc % 4 == 0
+  __device__ __forceinline__ int row(int m) const { return m; }
+  __device__ __forceinline__ int col(int n) const { return n; }
+  __device__ __forceinline__ void store(int m, int n, floatx4 v) const { store_c4(C, ldc, m, n, M, N, vec4, v); }
+};
+
+// relu(C) in 16 bits; N and ldc multiples of 4.
+template <typename T>
+struct StoreReluHalf {
+  uint16_t* C;
+  int ldc;
+  int M, N;
+  __device__ __forceinline__ int row(int m) const { return m; }
+  __device__ __forceinline__ int col(int n) const { return n; }
+  __device__ __forceinline__ void store(int m, int n, floatx4 v) const {
+    if (m < M && n < N) {
+      // (a comparison, as a NaN stays one)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = v[i] < 0.0f ? 0.0f : v[i];
+      }
+      u32x2 w;
+      w[0] = pack2<T>(v[0], v[1]);
+      w[1] = pack2<T>(v[2], v[3]);
+      *reinterpret_cast<u32x2*>(C + static_cast<size_t>(m) * ldc + n) = w;
+    }
+  }
+};
+
+// Row m = b T_ + t, column n = which E + h Dh + d of the QKV projection to Q
+// and K [b H + h][t][d] or V^T [b H + h][d][t]; Dh a multiple of 4.  A lane's
+// four columns are one 8-byte store to Q or K; to V^T, 16 lanes of a row block
+// write 32 contiguous bytes of each d.
+template <typename T>
+struct StoreQkv {
+  uint16_t* q;
+  uint16_t* k;
+  uint16_t* vt;
+  int M, T_, E, H, Dh, S_pad;
+  struct Row {
+    size_t image;  // b H S_pad Dh
+    int t;         // -1: past the last row
+  };
+  struct Col {
+    uint16_t* base;  // the head's part of Q, K or V^T
+    int d;
+    bool v;
+  };
+  __device__ __forceinline__ Row row(int m) const {
+    const int b = m / T_;
+    return {static_cast<size_t>(b) * H * S_pad * Dh, m < M ? m - b * T_ : -1};
+  }
+  __device__ __forceinline__ Col col(int n) const {
+    const int which = n / E;
+    const int r = n - which * E;
+    const int h = r / Dh;
+    return {(which == 0 ? q : which == 1 ? k : vt) + static_cast<size_t>(h) * S_pad * Dh, which < 3 ? r - h * Dh : -1,
+            which == 2};
+  }
+  __device__ __forceinline__ void store(const Row& r, const Col& c, floatx4 x) const {
+    if (r.t < 0 || c.d < 0) {
+      return;
+    }
+    u32x2 w;
+    w[0] = pack2<T>(x[0], x[1]);
+    w[1] = pack2<T>(x[2], x[3]);
+    uint16_t* p = c.base + r.image;
+    if (!c.v) {
+      *reinterpret_cast<u32x2*>(p + static_cast<size_t>(r.t) * Dh + c.d) = w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[static_cast<size_t>(c.d + i) * S_pad + r.t] = static_cast<uint16_t>(w[i >> 1] >> (16 * (i & 1)));
+      }
+    }
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Four waves in 2 x 2, each 16 RM x 16 CN of a 32 RM x 32 CN tile; LDS is a
 // ring of four 64-deep stages (128-byte rows, chunk c of row r at
@@ -27,16 +111,22 @@ namespace lchip::k {
 // 5.4 TB/s); 32x4096x8192 37 -> 13.0.  Sharing a tile's k range between two
 // workgroups gained only at 128x4096x4096 (13.8 -> 12.4 with 64x64, where the
 // 32x64 tile already takes 12.7), so tiles are never split.
+// The ViT block's GEMMs (M x 768 x 768, x 2304 for QKV) with these epilogues and
+// a separate attention kernel, against 128-row tiles of 12 stages of their own
+// and one kernel for QKV and attention (18.8 us already for one image, its
+// serial chain; 64 us for 32, three rounds): block of 224 x 224 images 30.9 ->
+// 18.8 us (batch 1), 32.7 -> 26.4 (4), 36.0 -> 33.9 (8), 67.7 -> 51 (16), 105.6
+// -> 93 (32); of 112 x 112 images 24.1 -> 17.3 (1), 25.3 -> 19.4 (8), 49.5 ->
+// 33.0 (32).
 // A has rows_a and Bt rows_b readable rows (tile rows past them read the last
 // one and are never stored); K is padded to 64; 32-bit lane offsets (the host
 // keeps 256 * ld * 2 bytes below 2^31).
 // ---------------------------------------------------------------------------
-template <typename T, int RM, int CN>
+template <typename T, int RM, int CN, typename Epi>
 __global__ __launch_bounds__(256) void gemm_half_tn_r4_kernel(const uint16_t* __restrict__ A,
-                                                              const uint16_t* __restrict__ Bt, float* __restrict__ C,
-                                                              int M, int N, int K, int rows_a, int rows_b,
-                                                              int lda, int ldb, int ldc, int tiles_m, int tiles_n,
-                                                              int vec4) {
+                                                              const uint16_t* __restrict__ Bt, int K, int rows_a,
+                                                              int rows_b, int lda, int ldb, int tiles_m, int tiles_n,
+                                                              Epi epi) {
   constexpr int BM = 32 * RM;
   constexpr int BN = 32 * CN;
   constexpr int NS = 4;
@@ -152,42 +242,50 @@ __global__ __launch_bounds__(256) void gemm_half_tn_r4_kernel(const uint16_t* __
     if (s + 3 < S) body(std::integral_constant<int, 3>{}, s + 3);
   }
   wait_vmcnt<0>();  // no copy may still be writing LDS
+  decltype(epi.col(0)) col[CN];
+#pragma unroll
+  for (int j = 0; j < CN; ++j) {
+    col[j] = epi.col(bn + 16 * (wn * CN + j) + 4 * lq);
+  }
 #pragma unroll
   for (int i = 0; i < RM; ++i) {
+    const auto row = epi.row(bm + 16 * (wm * RM + i) + lr);
 #pragma unroll
     for (int j = 0; j < CN; ++j) {
-      store_c4(C, ldc, bm + 16 * (wm * RM + i) + lr, bn + 16 * (wn * CN + j) + 4 * lq, M, N, vec4, acc[i][j]);
+      epi.store(row, col[j], acc[i][j]);
     }
   }
 }
 
-template <typename T, int RM, int CN>
-static hipError_t launch_r4(const uint16_t* A, const uint16_t* Bt, float* C, int M, int N, int K, int lda, int ldb,
-                            int ldc, hipStream_t stream) {
+template <typename T, int RM, int CN, typename Epi>
+static hipError_t launch_r4(const uint16_t* A, const uint16_t* Bt, int M, int N, int K, int lda, int ldb, Epi epi,
+                            hipStream_t stream) {
   const int tiles_m = (M + 32 * RM - 1) / (32 * RM);
   const int tiles_n = (N + 32 * CN - 1) / (32 * CN);
-  const int vec4 = (ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0) ? 1 : 0;
-  hipLaunchKernelGGL((gemm_half_tn_r4_kernel<T, RM, CN>), dim3(tiles_m * tiles_n), dim3(256), 0, stream, A, Bt,
-                     C, M, N, K, (M + kern::kHalfGemmBM - 1) / kern::kHalfGemmBM * kern::kHalfGemmBM,
-                     (N + kern::kHalfGemmBN - 1) / kern::kHalfGemmBN * kern::kHalfGemmBN, lda, ldb, ldc, tiles_m,
-                     tiles_n, vec4);
+  hipLaunchKernelGGL((gemm_half_tn_r4_kernel<T, RM, CN, Epi>), dim3(tiles_m * tiles_n), dim3(256), 0, stream, A, Bt, K,
+                     (M + kern::kHalfGemmBM - 1) / kern::kHalfGemmBM * kern::kHalfGemmBM,
+                     (N + kern::kHalfGemmBN - 1) / kern::kHalfGemmBN * kern::kHalfGemmBN, lda, ldb, tiles_m, tiles_n,
+                     epi);
   return hipGetLastError();
 }
 
-template <typename T>
-static hipError_t launch_r4_variant(kern::GemmHalfVariant v, const uint16_t* A, const uint16_t* Bt, float* C, int M,
-                                    int N, int K, int lda, int ldb, int ldc, hipStream_t stream) {
+template <typename T, typename Epi>
+static hipError_t launch_r4_variant(kern::GemmHalfVariant v, const uint16_t* A, const uint16_t* Bt, int M, int N, int K,
+                                    int lda, int ldb, Epi epi, hipStream_t stream) {
+  if (K <= 0 || K % kern::kHalfGemmBK != 0 || M <= 0 || N <= 0 || !kern::gemmHalfR4Fits(lda, ldb)) {
+    return hipErrorInvalidValue;
+  }
   switch (v) {
     case kern::GemmHalfVariant::kR128:
-      return launch_r4<T, 4, 4>(A, Bt, C, M, N, K, lda, ldb, ldc, stream);
+      return launch_r4<T, 4, 4>(A, Bt, M, N, K, lda, ldb, epi, stream);
     case kern::GemmHalfVariant::kR96:
-      return launch_r4<T, 3, 4>(A, Bt, C, M, N, K, lda, ldb, ldc, stream);
+      return launch_r4<T, 3, 4>(A, Bt, M, N, K, lda, ldb, epi, stream);
     case kern::GemmHalfVariant::kR64x128:
-      return launch_r4<T, 2, 4>(A, Bt, C, M, N, K, lda, ldb, ldc, stream);
+      return launch_r4<T, 2, 4>(A, Bt, M, N, K, lda, ldb, epi, stream);
     case kern::GemmHalfVariant::kR64:
-      return launch_r4<T, 2, 2>(A, Bt, C, M, N, K, lda, ldb, ldc, stream);
+      return launch_r4<T, 2, 2>(A, Bt, M, N, K, lda, ldb, epi, stream);
     case kern::GemmHalfVariant::kR32:
-      return launch_r4<T, 1, 2>(A, Bt, C, M, N, K, lda, ldb, ldc, stream);
+      return launch_r4<T, 1, 2>(A, Bt, M, N, K, lda, ldb, epi, stream);
     default:
       return hipErrorInvalidValue;
   }
@@ -229,12 +327,35 @@ GemmHalfVariant gemmHalfR4Choose(int M, int N, int K, int cus) {
 
 hipError_t gemmHalfR4(const uint16_t* A, const uint16_t* Bt, float* C, int M, int N, int K, int lda, int ldb, int ldc,
                       Half t, GemmHalfVariant variant, hipStream_t stream) {
-  if (K <= 0 || K % kHalfGemmBK != 0 || M <= 0 || N <= 0 || !gemmHalfR4Fits(lda, ldb)) {
+  const int vec4 = (ldc % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0) ? 1 : 0;
+  const k::StoreF32 epi{C, ldc, M, N, vec4};
+  return t == Half::kBF16 ? k::launch_r4_variant<k::BF16>(variant, A, Bt, M, N, K, lda, ldb, epi, stream)
+                          : k::launch_r4_variant<k::F16>(variant, A, Bt, M, N, K, lda, ldb, epi, stream);
+}
+
+hipError_t gemmHalfR4Relu(const uint16_t* A, const uint16_t* Bt, uint16_t* C, int M, int N, int K, int lda, int ldb,
+                          int ldc, Half t, int cus, hipStream_t stream) {
+  if (N % 4 != 0 || ldc % 4 != 0) {
     return hipErrorInvalidValue;
   }
+  const GemmHalfVariant v = gemmHalfR4Choose(M, N, K, cus);
   return t == Half::kBF16
-             ? k::launch_r4_variant<k::BF16>(variant, A, Bt, C, M, N, K, lda, ldb, ldc, stream)
-             : k::launch_r4_variant<k::F16>(variant, A, Bt, C, M, N, K, lda, ldb, ldc, stream);
+             ? k::launch_r4_variant<k::BF16>(v, A, Bt, M, N, K, lda, ldb, k::StoreReluHalf<k::BF16>{C, ldc, M, N}, stream)
+             : k::launch_r4_variant<k::F16>(v, A, Bt, M, N, K, lda, ldb, k::StoreReluHalf<k::F16>{C, ldc, M, N}, stream);
+}
+
+hipError_t gemmHalfR4Qkv(const uint16_t* tokens, const uint16_t* Wqkv_t, uint16_t* q, uint16_t* k_, uint16_t* vt, int B,
+                         int T_, int E, int H, int S_pad, Half t, int cus, hipStream_t stream) {
+  const int M = B * T_;
+  const int Dh = E / H;
+  if (E % H != 0 || Dh % 4 != 0) {
+    return hipErrorInvalidValue;
+  }
+  const GemmHalfVariant v = gemmHalfR4Choose(M, 3 * E, E, cus);
+  return t == Half::kBF16 ? k::launch_r4_variant<k::BF16>(v, tokens, Wqkv_t, M, 3 * E, E, E, E,
+                                                          k::StoreQkv<k::BF16>{q, k_, vt, M, T_, E, H, Dh, S_pad}, stream)
+                          : k::launch_r4_variant<k::F16>(v, tokens, Wqkv_t, M, 3 * E, E, E, E,
+                                                         k::StoreQkv<k::F16>{q, k_, vt, M, T_, E, H, Dh, S_pad}, stream);
 }
 
 }  // namespace lchip::kern

@@ -322,10 +322,11 @@ def bench_config2(lc, synth, cpu):
         per_call.append(time.perf_counter() - t0)
     per_call.sort()
     entry["one_shot_ms_per_call_1024^3"] = round(per_call[len(per_call) // 2] * 1e3, 5)
-    entry["kernel_1024^3"] = {"kernel": "gemm_f32_lds_kernel<64,2,2> (v_mfma_f32_32x32x2_f32)",
+    variant, kernel_fn = sess[0].kernel_name().split()
+    entry["kernel_1024^3"] = {"kernel": f"{kernel_fn} ({variant})",
                               "avg_kernel_ms": round(kms, 5), "TFLOP/s": round(achieved, 3),
                               "frac_peak": round(achieved / PEAK_TFLOPS["f32"], 4),
-                              "traffic": GEMM_F32_1024_TRAFFIC}
+                              "traffic": GEMM_F32_1024_TRAFFIC.get(kernel_fn)}
     if cpu.kind is not None:
         t0 = time.perf_counter()
         reps_done, flops_done = 0, 0.0
@@ -563,7 +564,8 @@ PMC_COPIES = 10
 PMC_GEMMS = 20
 # FETCH_SIZE: GEMM 12329.9 KiB/dispatch, copy 131084.4 KiB for 262144 KiB moved (x2.000);
 # WRITE_SIZE: GEMM 4096.0 KiB/dispatch, copy 262144.0 KiB (x1.000).
-GEMM_F32_1024_TRAFFIC = 25235186 + 4194304  # HBM bytes per launch (fetch + write, calibrated)
+# HBM bytes per launch (fetch + write, calibrated); other kernels report null.
+GEMM_F32_1024_TRAFFIC = {"gemm_f32_lds_kernel": 25235186 + 4194304}
 # 8192^3 bf16, HBM bytes per launch (fetch + write, calibrated), per kernel:
 # profiles/gemm_half_tn_w4h_kernel_8192cube_traffic.txt: FETCH_SIZE 787628.8 KiB/dispatch (x1.9998),
 # WRITE_SIZE 262144.0 KiB (x1.000).  A kernel without its own counter passes (a variant forced by

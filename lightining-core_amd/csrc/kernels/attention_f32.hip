@@ -164,6 +164,11 @@ __global__ __launch_bounds__(256 * KG, DK <= 2 ? 2 : 1) void attn_fwd_f32_split_
     t1 = min(t1, t0 + split_tiles);
   }
   const int n = (t1 - t0 + KG - 1) / KG;  // iterations; iteration t: tile t0 + t * KG + kg
+  // The wave's last tile: up to its queries' diagonal.  Only that tile can need
+  // masks (queries and tiles are both cut at multiples of 32), so a non-finite V
+  // row reaches no query before its own tile.
+  const int edge_tile = causal ? min(nt - 1, q0 / 32) : nt - 1;
+  const int last_tile = min(edge_tile, t1 - 1);
 
   floatx4 o[2][DB], ol[2][DB];  // hh products; the small ones
   float m_run[2], l_run[2];
@@ -233,7 +238,7 @@ __global__ __launch_bounds__(256 * KG, DK <= 2 ? 2 : 1) void attn_fwd_f32_split_
   if (*in.guard == in.epoch) {
     // the fp32 operands, straight from memory
     const size_t base = static_cast<size_t>(head) * S * D;
-    for (int t = t0 + kg; t < t1; t += KG) {
+    for (int t = t0 + kg; t <= last_tile; t += KG) {
       const int j0 = t * 32;
       floatx4 st[2][2];
 #pragma unroll
@@ -302,10 +307,6 @@ __global__ __launch_bounds__(256 * KG, DK <= 2 ? 2 : 1) void attn_fwd_f32_split_
     typedef __attribute__((address_space(3))) const char lds_char;
     typedef __attribute__((address_space(3))) const u32x4 lds_u32x4;
     lds_char* lbase = (lds_char*)(smem) + kg * 3 * TILE + lane * 16;
-    // The wave's last tile: up to its queries' diagonal.  Only the last one can
-    // need masks (queries and tiles are both cut at multiples of 32).
-    const int last_tile = min(causal ? min(nt - 1, q0 / 32) : nt - 1, t1 - 1);
-    const int edge_tile = causal ? min(nt - 1, q0 / 32) : nt - 1;
     auto scores = [&](int slot, floatx4 (&st)[2][2]) {
       lds_char* tile = lbase + slot * TILE;
 #pragma unroll

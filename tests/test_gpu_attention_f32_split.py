@@ -94,9 +94,7 @@ def test_operands_outside_the_split(lc, b, h, s, d, what):
         k *= np.float32(1e33)
     else:
         v *= np.float32(1e30)
-    # causal only where every value is finite: a later key's infinity meets a
-    # query as 0 * inf only within the query's own tile
-    causal = what in ("tiny", "huge")
+    causal = what in ("tiny", "huge")  # non-finite values and masks: the next test
     ref = _reference(q, k, v, causal)
     sess = lc.AttentionSession.batched(b, h, s, d, causal=causal, compute_dtype="f32")
     first, later = np.empty(q.size, np.float32), np.empty(q.size, np.float32)
@@ -109,3 +107,31 @@ def test_operands_outside_the_split(lc, b, h, s, d, what):
         np.testing.assert_array_equal(np.where(fine, 0.0, got), np.where(fine, 0.0, ref.ravel()))
         assert np.all(np.isfinite(got[fine]))
         assert np.linalg.norm(got[fine] - ref.ravel()[fine]) <= TOL * np.linalg.norm(ref.ravel()[fine])
+
+
+# (heads, S, D): two key groups with and without key splits, one group (D = 128)
+# with and without, enough blocks for none of either
+@pytest.mark.parametrize("h,s,d", [(9, 520, 64), (9, 1025, 64), (70, 160, 64), (2, 200, 128), (1, 600, 128),
+                                   (40, 300, 128)])
+@pytest.mark.parametrize("what", ["nan", "inf"])
+@pytest.mark.parametrize("key", [33, 100, 127])
+def test_causal_non_finite_value_stays_behind_its_tile(lc, h, s, d, what, key):
+    """A non-finite V row meets a masked query as 0 * inf only within the query's
+    own 32 keys: every earlier row is finite, whether the kernel finds the value
+    (first call) or the host has seen it (later calls)."""
+    q, k, v = _inputs((1, h, s, d))
+    ref = _reference(q, k, v, True)[0]
+    v[0, 0, key, 3] = np.nan if what == "nan" else np.inf
+    sess = lc.AttentionSession.batched(1, h, s, d, causal=True, compute_dtype="f32")
+    first, later = np.empty(q.size, np.float32), np.empty(q.size, np.float32)
+    sess.forward_with_policy_into(q, k, v, first, lc.AttentionIoPolicy())
+    sess.forward_with_policy_into(q, k, v, later, lc.AttentionIoPolicy(upload_q=False, upload_k=False,
+                                                                       upload_v=False))
+    sess.close()
+    assert np.array_equal(np.isfinite(first), np.isfinite(later))
+    tile = key // 32 * 32
+    for got in (first.reshape(h, s, d), later.reshape(h, s, d)):
+        assert not np.isfinite(got[0, key:, 3]).any()  # a query that sees the value
+        got[0, tile:, 3] = ref[0, tile:, 3]
+        assert np.isfinite(got).all()
+        assert np.linalg.norm(got - ref) <= TOL * np.linalg.norm(ref)

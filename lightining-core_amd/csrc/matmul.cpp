@@ -183,38 +183,74 @@ VariantTable variants(bool half) {
               : VariantTable{std::begin(kF32Variants), std::end(kF32Variants)};
 }
 
-TuneEntry entryFor(bool half, int variant) {
-  TuneEntry e;
+const VariantInfo* infoOf(bool half, int variant) {
   for (const VariantInfo& v : variants(half)) {
     if (v.variant == variant) {
-      e.kernel = v.name;
-      e.tile_m = v.tile_m;
-      e.tile_n = v.tile_n;
-      e.tile_k = v.tile_k;
-      e.waves = v.waves;
-      e.split_k = v.split_k;
+      return &v;
     }
   }
+  return nullptr;
+}
+
+bool isSplit(int variant) { return variant >= static_cast<int>(kern::GemmF32Variant::kSplit64); }
+
+// The variants of a shape (0: not settled).  fp32 has two: `once` for a call
+// that uploads an operand and launches once, never one of the split GEMM, and
+// `resident` for every other launch.  The tune cache's row names one variant
+// for both ("A"), or "once|resident", or "once|" before a resident launch was
+// timed; a row that names a split variant alone leaves `once` open.
+struct Choices {
+  int once = 0;
+  int resident = 0;
+};
+
+TuneEntry entryFor(bool half, const Choices& c) {
+  const VariantInfo* once = infoOf(half, c.once);
+  const VariantInfo* resident = infoOf(half, c.resident);
+  const VariantInfo* v = resident != nullptr ? resident : once;  // the row's figures
+  TuneEntry e;
+  e.kernel = c.once == c.resident ? v->name
+                                  : std::string(once->name) + "|" + (resident != nullptr ? resident->name : "");
+  e.tile_m = v->tile_m;
+  e.tile_n = v->tile_n;
+  e.tile_k = v->tile_k;
+  e.waves = v->waves;
+  e.split_k = v->split_k;
   return e;
 }
 
-// A cached entry names a variant this shape can run (else it is ignored).
-bool variantFromEntry(const TuneEntry& e, bool half, std::size_t m, std::size_t k, int* variant) {
+// The variant a cached row names, 0 unless this shape can run it.
+int variantFromName(const std::string& name, bool half, std::size_t m, std::size_t k) {
   const long long k_pad = static_cast<long long>(roundUp(k, kern::kHalfGemmBK));
   for (const VariantInfo& v : variants(half)) {
-    if (e.kernel == v.name) {
+    if (name == v.name) {
       const bool skinny = v.variant == static_cast<int>(kern::GemmHalfVariant::kSkinny);
       if (half && skinny != (m <= 16)) {
-        return false;
+        return 0;
       }
       if (half && kern::isR4(static_cast<kern::GemmHalfVariant>(v.variant)) && !kern::gemmHalfR4Fits(k_pad, k_pad)) {
-        return false;
+        return 0;
       }
-      *variant = v.variant;
-      return true;
+      return v.variant;
     }
   }
-  return false;
+  return 0;
+}
+
+Choices cachedChoices(HipContext* ctx, const MatMulResident& r) {
+  const bool half = isHalf(r.dtype);
+  Choices c;
+  TuneEntry e;
+  if (!tuneLookup(r.m, r.k, r.n, static_cast<int>(r.dtype), baseArch(ctx), &e)) {
+    return c;
+  }
+  const std::size_t bar = e.kernel.find('|');
+  c.once = variantFromName(e.kernel.substr(0, bar), half, r.m, r.k);
+  c.resident = bar == std::string::npos ? c.once : variantFromName(e.kernel.substr(bar + 1), half, r.m, r.k);
+  if (!half && isSplit(c.once)) {
+    c.once = 0;
+  }
+  return c;
 }
 
 int cuCount(const HipContext* ctx) {
@@ -229,8 +265,6 @@ bool splitFits(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t 
   const std::size_t rows = roundUp(m, kern::kF32GemmBM) + roundUp(n, kern::kF32GemmBN);
   return kp <= (std::size_t{1} << 23) && 3 * sizeof(uint16_t) * rows * kp <= ctx->props.totalGlobalMem / 8;
 }
-
-bool isSplit(int variant) { return variant >= static_cast<int>(kern::GemmF32Variant::kSplit64); }
 
 // The GEMM of a split variant (its planes made first if they are stale);
 // false when its buffers cannot be had, and nothing was launched.
@@ -290,7 +324,7 @@ hipError_t launchGemm(HipContext* ctx, MatMulResident& r, int variant) {
           launchSplitGemm(ctx, r, static_cast<kern::GemmF32Variant>(variant), &e)) {
         return e;
       }
-      variant = static_cast<int>(kern::GemmF32Variant::kAuto);
+      variant = r.once;
     }
     // stream-K: one workgroup per CU (a whole-tile grid may hold two per CU)
     const int groups = cuCount(ctx);
@@ -400,22 +434,85 @@ int defaultHalfVariant(const HipContext* ctx, std::size_t m, std::size_t k, std:
   return static_cast<int>(v);
 }
 
-// Settles r.variant for the shape: a tune-cache entry, else (CJ_MATMUL_AUTOTUNE
-// not off) the fastest candidate, else the heuristic; the choice is recorded.
-// CJ_HIP_GEMM_F32 / CJ_HIP_GEMM_TILE (sweep overrides) bypass all of it.
+bool forcedVariant(bool half) { return std::getenv(half ? "CJ_HIP_GEMM_TILE" : "CJ_HIP_GEMM_F32") != nullptr; }
+
+// `preferred` (the heuristic's choice) unless another candidate is clearly
+// faster (3%: below that the measurement cannot tell them apart); candidates
+// past `accept` do not count.
+template <typename Accept>
+int fastest(const std::vector<int>& cands, const std::vector<float>& ms, int preferred, Accept accept) {
+  float ref_ms = 0.0f;
+  for (std::size_t c = 0; c < ms.size(); ++c) {
+    if (cands[c] == preferred) {
+      ref_ms = ms[c];
+    }
+  }
+  int best = preferred;
+  float best_ms = ref_ms > 0.0f ? ref_ms * 0.97f : 0.0f;
+  for (std::size_t c = 0; c < ms.size(); ++c) {
+    if (accept(cands[c]) && (best_ms <= 0.0f || ms[c] < best_ms)) {
+      best_ms = ms[c];
+      best = cands[c];
+    }
+  }
+  return best;
+}
+
+int defaultOnceVariant(const HipContext* ctx, const MatMulResident& r) {
+  return static_cast<int>(kern::gemmF32Choose(static_cast<int>(r.m), static_cast<int>(r.n), cuCount(ctx)));
+}
+
+void recordChoices(HipContext* ctx, const MatMulResident& r, const Choices& c) {
+  if (infoOf(isHalf(r.dtype), c.once) == nullptr) {
+    return;
+  }
+  tuneRecord(r.m, r.k, r.n, static_cast<int>(r.dtype), baseArch(ctx), entryFor(isHalf(r.dtype), c));
+}
+
+// Settles r.once (fp32): a tune-cache entry, else (CJ_MATMUL_AUTOTUNE not off)
+// the faster of whole tiles and stream-K, else the heuristic; the choice is
+// recorded.  CJ_HIP_GEMM_F32 (a sweep override) bypasses all of it.
+Status settleOnce(HipContext* ctx, MatMulResident& r) {
+  if (r.once_tuned) {
+    return Status::kSuccess;
+  }
+  r.once = 0;
+  if (!forcedVariant(false)) {
+    Choices c = cachedChoices(ctx, r);
+    if (c.once == 0) {
+      const std::vector<int> cands = {static_cast<int>(kern::GemmF32Variant::kDataParallel),
+                                      static_cast<int>(kern::GemmF32Variant::kStreamK)};
+      std::vector<float> ms;
+      if (autotuneEnabled("CJ_MATMUL_AUTOTUNE")) {
+        LC_TRY(timeVariants(ctx, r, cands, &ms));
+      }
+      c.once = fastest(cands, ms, defaultOnceVariant(ctx, r), [](int) { return true; });
+      recordChoices(ctx, r, c);
+    }
+    r.once = c.once;
+  }
+  r.once_tuned = true;
+  return Status::kSuccess;
+}
+
+// Settles r.variant likewise, over every candidate for the shape and dtype.
+// CJ_HIP_GEMM_F32 / CJ_HIP_GEMM_TILE bypass it.
 Status settleVariant(HipContext* ctx, MatMulResident& r) {
+  if (r.tuned) {
+    return Status::kSuccess;
+  }
   const bool half = isHalf(r.dtype);
   r.variant = 0;
-  if (std::getenv(half ? "CJ_HIP_GEMM_TILE" : "CJ_HIP_GEMM_F32") != nullptr) {
+  if (forcedVariant(half)) {
+    r.tuned = true;
     return Status::kSuccess;
   }
-  const std::string arch = baseArch(ctx);
-  const int dtype = static_cast<int>(r.dtype);
-  TuneEntry known;
-  if (tuneLookup(r.m, r.k, r.n, dtype, arch, &known) && variantFromEntry(known, half, r.m, r.k, &r.variant)) {
+  Choices c = cachedChoices(ctx, r);
+  if (c.resident != 0) {
+    r.variant = c.resident;
+    r.tuned = true;
     return Status::kSuccess;
   }
-  int best = half ? defaultHalfVariant(ctx, r.m, r.k, r.n) : defaultF32Variant(ctx, r.m, r.k, r.n);
   std::vector<int> cands;
   if (!half) {
     cands = {static_cast<int>(kern::GemmF32Variant::kDataParallel), static_cast<int>(kern::GemmF32Variant::kStreamK)};
@@ -436,39 +533,41 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
       }
     }
   }
+  std::vector<float> ms;
   if (cands.size() > 1 && autotuneEnabled("CJ_MATMUL_AUTOTUNE")) {
-    std::vector<float> ms;
     LC_TRY(timeVariants(ctx, r, cands, &ms));
-    // The heuristic's choice stays unless another variant is clearly faster
-    // (3%: below that the measurement cannot tell them apart).
-    float ref_ms = 0.0f;
-    for (std::size_t c = 0; c < cands.size(); ++c) {
-      if (cands[c] == best) {
-        ref_ms = ms[c];
-      }
-    }
-    float best_ms = ref_ms > 0.0f ? ref_ms * 0.97f : 0.0f;
-    for (std::size_t c = 0; c < cands.size(); ++c) {
-      if (best_ms <= 0.0f || ms[c] < best_ms) {
-        best_ms = ms[c];
-        best = cands[c];
-      }
-    }
   }
-  r.variant = best;
-  tuneRecord(r.m, r.k, r.n, dtype, arch, entryFor(half, best));
+  c.resident = fastest(cands, ms, half ? defaultHalfVariant(ctx, r.m, r.k, r.n) : defaultF32Variant(ctx, r.m, r.k, r.n),
+                       [](int) { return true; });
+  if (half) {
+    c.once = c.resident;
+  } else if (c.once == 0) {
+    c.once = fastest(cands, ms, defaultOnceVariant(ctx, r), [](int v) { return !isSplit(v); });
+  }
+  recordChoices(ctx, r, c);
+  r.variant = c.resident;
+  r.tuned = true;
   return Status::kSuccess;
 }
 
-// The variant for a call that uploads an fp32 operand and launches once: the
-// planes of a new operand cost 5 us (256^3) to 12 us (2048^3), more than the
-// split GEMM saves below 2^32 products (1024^3: 6.4 + 16.1 us against 22.3).
-int oneShotVariant(const MatMulResident& r) {
-  const bool stale = !r.has_planes_a || !r.has_planes_b;
-  if (!isHalf(r.dtype) && isSplit(r.variant) && stale && r.m * r.k * r.n < (std::size_t{1} << 32)) {
-    return static_cast<int>(kern::GemmF32Variant::kAuto);
+// The variant of a launch.  A call that uploads an fp32 operand and launches
+// once keeps the fp32 instruction below 2^32 products: the planes of a new
+// operand cost 5 us (256^3) to 12 us (2048^3), more than the split GEMM saves
+// there (1024^3: 6.4 + 16.1 us against 22.3).  That depends on the call alone,
+// so equal calls give equal bits whatever ran before them.
+Status launchVariant(HipContext* ctx, MatMulResident& r, bool one_shot, int* variant) {
+  if (one_shot && !isHalf(r.dtype) && r.m * r.k * r.n < (std::size_t{1} << 32)) {
+    LC_TRY(settleOnce(ctx, r));
+    *variant = r.once;
+    return Status::kSuccess;
   }
-  return r.variant;
+  LC_TRY(settleVariant(ctx, r));
+  *variant = r.variant;
+  if (!isHalf(r.dtype) && isSplit(r.variant) && knownUnsafe(ctx, r)) {
+    LC_TRY(settleOnce(ctx, r));
+    *variant = r.once;
+  }
+  return Status::kSuccess;
 }
 
 // Small fp32 calls that upload both operands and download the product (the
@@ -516,16 +615,14 @@ Status matmulQuick(HipContext* ctx, MatMulResident& r, const float* a, const flo
     return failHip(e, "matmul upload padding");
   }
   r.has_a = r.has_b = true;
-  if (!r.tuned) {
-    LC_TRY(settleVariant(ctx, r));
-    r.tuned = true;
-  }
+  int variant = 0;
+  LC_TRY(launchVariant(ctx, r, true, &variant));
   unsigned* flag_dev = nullptr;
   unsigned* count_dev = nullptr;
   unsigned seq = 0;
   LC_TRY(prepareDoneFlag(ctx, &flag_dev, &count_dev, &seq));
   traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, r.m * r.k * r.n);
-  e = launchGemm(ctx, r, oneShotVariant(r));
+  e = launchGemm(ctx, r, variant);
   if (e != hipSuccess) {
     return failHip(e, "matmul kernel launch");
   }
@@ -557,7 +654,8 @@ Status matmulResident(HipContext* ctx, MatMulResident& r, std::size_t m, std::si
   }
   if (r.m != m || r.k != k || r.n != n || r.dtype != dtype) {
     r.has_a = r.has_b = r.has_c = false;
-    r.tuned = false;
+    r.tuned = r.once_tuned = false;
+    r.variant = r.once = 0;
     r.m = m;
     r.k = k;
     r.n = n;
@@ -580,12 +678,11 @@ Status matmulResident(HipContext* ctx, MatMulResident& r, std::size_t m, std::si
   }
   LC_TRY(r.c.ensure(m * n * sizeof(float)));
   const std::size_t hint = m * k * n;
-  if (!r.tuned && repeat > 0) {
-    LC_TRY(settleVariant(ctx, r));
-    r.tuned = true;
+  int variant = 0;
+  if (repeat > 0) {
+    const bool one_shot = repeat == 1 && policy.download_out && (policy.upload_a || policy.upload_b);
+    LC_TRY(launchVariant(ctx, r, one_shot, &variant));
   }
-  const bool one_shot = repeat == 1 && policy.download_out && (policy.upload_a || policy.upload_b);
-  const int variant = one_shot ? oneShotVariant(r) : r.variant;
   for (std::size_t i = 0; i < repeat; ++i) {
     traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, hint);
     const hipError_t e = launchGemm(ctx, r, variant);
@@ -781,12 +878,10 @@ lcError_t lcMatMulResidentSessionTimeLaunches(lcMatMulResidentSession* s, size_t
   if (!r.has_a || !r.has_b || r.m != s->m || r.k != s->k || r.n != s->n || r.dtype != s->dtype) {
     return toLc(fail(Status::kInvalidValue, "matmul session: no resident inputs to time (start the session first)"));
   }
-  if (!r.tuned) {
-    st = settleVariant(ctx, r);
-    if (st != Status::kSuccess) {
-      return toLc(st);
-    }
-    r.tuned = true;
+  int variant = 0;
+  st = launchVariant(ctx, r, false, &variant);
+  if (st != Status::kSuccess) {
+    return toLc(st);
   }
   std::vector<hipEvent_t> ev(2 * count, nullptr);
   hipError_t e = hipSuccess;
@@ -797,7 +892,7 @@ lcError_t lcMatMulResidentSessionTimeLaunches(lcMatMulResidentSession* s, size_t
     e = hipEventRecord(ev[2 * i], ctx->stream);
     if (e == hipSuccess) {
       traceOpDispatch(TraceOp::kMatMul, Device::kHIP, Device::kHIP, false, r.m * r.k * r.n);
-      e = launchGemm(ctx, r, r.variant);
+      e = launchGemm(ctx, r, variant);
     }
     if (e == hipSuccess) {
       e = hipEventRecord(ev[2 * i + 1], ctx->stream);

@@ -87,6 +87,10 @@ struct MatMulResident {
   // the first launch from the tune cache, an autotune or the heuristic.
   int variant = 0;
   bool tuned = false;
+  // fp32: the same for a call that uploads an operand and launches once, and for
+  // operands the split GEMM does not take.
+  int once = 0;
+  bool once_tuned = false;
   // fp32: the bf16 parts of A, then of B (kern::SplitOperandF32), made when a
   // split GEMM first needs them after an upload.
   DeviceBuffer planes;

@@ -9,8 +9,10 @@
 namespace lchip {
 
 // One GEMM configuration.  `kernel` names the variant ("f32_dp_64x64x64",
-// "half_lds_256x256", ...); the tile / wave / split fields describe it for a
-// reader of the cache file.
+// "half_lds_256x256", ...), or two of an fp32 shape, "once|resident": the one
+// for calls that upload an operand and launch once, then the one for resident
+// launches (empty: not timed yet).  The tile / wave / split fields describe the
+// last one named for a reader of the cache file.
 struct TuneEntry {
   std::string kernel;
   int tile_m = 0;

@@ -133,3 +133,39 @@ def test_guard_follows_each_upload(lc):
         assert np.array_equal(fin, np.isfinite(got)) and np.array_equal(got[~fin], ref[~fin].astype(np.float32))
         assert np.abs(got[fin] - ref[fin]).max() <= 1e-5 * np.abs(ref[fin]).max()
     s.close()
+
+
+def test_plain_calls_do_not_depend_on_what_ran_before(lc, tmp_path):
+    """Equal matmul2d calls give equal bits: the first of a shape, a later one,
+    one after a resident session has timed the split variants, and one in a
+    process that finds the tune cache of the first; below 2^32 products none of
+    them runs a split variant, and the session still does where it is faster."""
+    shapes = [(600, 700, 500), (640, 2048, 640), (1000, 777, 1030), (64, 64, 64)]
+    body = f"""
+        import hashlib
+        import sys
+        import lightning_core as lc
+        from lightning_core import synth
+        for m, k, n in {shapes!r}:
+            print("[case]", m, k, n, flush=True)
+            a, b = synth.normal((m, k), stream=61), synth.normal((k, n), stream=62)
+            calls = [lc.matmul2d(a, b) for _ in range(3)]
+            s = lc.MatMulResidentSession(m, k, n)
+            s.start_into(a, b)
+            s.finish_into()
+            name = s.kernel_name()
+            s.close()
+            calls.append(lc.matmul2d(a, b))
+            print("SHA", m, k, n, name.split()[0], *(hashlib.sha256(c.tobytes()).hexdigest() for c in calls), flush=True)
+    """
+    rows = [[line.split()[1:] for line in _child(body, tmp_path).splitlines() if line.startswith("SHA")]
+            for _ in range(2)]
+    cached = [r.split(",") for r in (tmp_path / ".lightning_core_matmul_tune_cache.csv").read_text().splitlines()
+              if not r.startswith("#")]
+    assert len(rows[0]) == len(shapes) == len(cached)
+    for first, again in zip(*rows):
+        assert len(set(first[4:] + again[4:])) == 1, first[:3]
+        assert first[3] == again[3]  # the session's variant comes from the cache
+        once, _, resident = next(r[5] for r in cached if r[:3] == first[:3]).partition("|")
+        assert "split" not in once and (resident or once) == first[3]
+    assert any("split" in r[3] for r in rows[0])

@@ -513,10 +513,21 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
     r.tuned = true;
     return Status::kSuccess;
   }
+  const bool timed = autotuneEnabled("CJ_MATMUL_AUTOTUNE");
   std::vector<int> cands;
   if (!half) {
     cands = {static_cast<int>(kern::GemmF32Variant::kDataParallel), static_cast<int>(kern::GemmF32Variant::kStreamK)};
     if (splitFits(ctx, r.m, r.k, r.n)) {
+      if (timed) {
+        // A split variant's time is that of operands it takes.  With others (the
+        // scans of both have run after this sync) nothing is settled or recorded.
+        LC_TRY(syncStream(ctx));
+        if (knownUnsafe(ctx, r)) {
+          LC_TRY(settleOnce(ctx, r));
+          r.variant = r.once;
+          return Status::kSuccess;
+        }
+      }
       for (const VariantInfo& v : kF32Variants) {
         if (isSplit(v.variant)) {
           cands.push_back(v.variant);
@@ -534,7 +545,7 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
     }
   }
   std::vector<float> ms;
-  if (cands.size() > 1 && autotuneEnabled("CJ_MATMUL_AUTOTUNE")) {
+  if (cands.size() > 1 && timed) {
     LC_TRY(timeVariants(ctx, r, cands, &ms));
   }
   c.resident = fastest(cands, ms, half ? defaultHalfVariant(ctx, r.m, r.k, r.n) : defaultF32Variant(ctx, r.m, r.k, r.n),
@@ -561,12 +572,13 @@ Status launchVariant(HipContext* ctx, MatMulResident& r, bool one_shot, int* var
     *variant = r.once;
     return Status::kSuccess;
   }
-  LC_TRY(settleVariant(ctx, r));
-  *variant = r.variant;
-  if (!isHalf(r.dtype) && isSplit(r.variant) && knownUnsafe(ctx, r)) {
+  if (!isHalf(r.dtype) && knownUnsafe(ctx, r) && (!r.tuned || isSplit(r.variant))) {
     LC_TRY(settleOnce(ctx, r));
     *variant = r.once;
+    return Status::kSuccess;
   }
+  LC_TRY(settleVariant(ctx, r));
+  *variant = r.variant;
   return Status::kSuccess;
 }
 

@@ -169,3 +169,37 @@ def test_plain_calls_do_not_depend_on_what_ran_before(lc, tmp_path):
         once, _, resident = next(r[5] for r in cached if r[:3] == first[:3]).partition("|")
         assert "split" not in once and (resident or once) == first[3]
     assert any("split" in r[3] for r in rows[0])
+
+
+def test_unfit_operands_settle_no_split_choice(lc, tmp_path):
+    """The choice of a resident launch's variant is timed on operands the split
+    GEMM takes: a session that starts with one it does not take leaves it open,
+    in the session and in the tune cache, and the next fit upload settles it."""
+    cache = tmp_path / ".lightning_core_matmul_tune_cache.csv"
+    out = _child(f"""
+        import numpy as np
+        import lightning_core as lc
+        from lightning_core import synth
+        def row():
+            return next(r.split(",")[5] for r in open({str(cache)!r}) if r.startswith("640,2048,640,"))
+        m, k, n = 640, 2048, 640
+        a, b = synth.normal((m, k), stream=71), synth.normal((k, n), stream=72)
+        bad = a.copy()
+        bad[1, 2] = 1e-35
+        s = lc.MatMulResidentSession(m, k, n)
+        for _ in range(2):
+            s.start_into(bad, b)
+            c = s.finish_into().reshape(m, n)
+            assert np.abs(c - bad.astype(np.float64) @ b).max() <= 1e-4 * np.abs(c).max()
+            print("ROW", row(), flush=True)
+        s.start_into(a, b)
+        s.finish_into()
+        print("ROW", row(), s.kernel_name().split()[0], flush=True)
+        s.close()
+    """, tmp_path)
+    rows = [line.split()[1:] for line in out.splitlines() if line.startswith("ROW")]
+    for (name,) in rows[:2]:
+        once, bar, resident = name.partition("|")
+        assert bar and not resident and "split" not in once
+    name, kernel = rows[2]
+    assert name.partition("|")[2] == kernel and "split" in kernel

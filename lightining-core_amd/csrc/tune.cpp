@@ -7,6 +7,7 @@
 // version 2 is written; a header of another kind or version clears the table
 // (the reference re-tunes then).  Rows are re-keyed for gfx950:
 //   matmul    m,k,n,dtype,arch,kernel,tile_m,tile_n,tile_k,waves,split_k
+//             ("#columns" ends in the number of the autotune's variant set)
 //   attention HF|HT,seq,dim,causal,resident_hint,sync_hint,[compute_loss,]arch,splits
 // Rows in the reference's own layouts (matmul: 5 or 6 columns, Metal tiles;
 // attention: F / T rows whose mode is a Metal forward / train mode) mean
@@ -78,9 +79,10 @@ std::string pathFrom(const char* env, const char* fallback) {
 
 // Reads a cache file: returns false when it cannot be opened.  `header_ok`
 // is false when a tag line names another kind or an unsupported version;
-// `rows` receives every non-comment line split into columns.
+// `rows` receives every non-comment line split into columns, `columns` (unless
+// null) the file's "#columns" line.
 bool readCacheFile(const std::string& path, const char* kind, bool* header_ok,
-                   std::vector<std::vector<std::string>>* rows) {
+                   std::vector<std::vector<std::string>>* rows, std::string* columns = nullptr) {
   std::ifstream f(path);
   if (!f.is_open()) {
     return false;
@@ -108,6 +110,8 @@ bool readCacheFile(const std::string& path, const char* kind, bool* header_ok,
           *header_ok = false;
           return true;
         }
+      } else if (cols[0] == "#columns" && columns != nullptr) {
+        *columns = t;
       }
       continue;
     }
@@ -134,14 +138,23 @@ MatmulCache& mm() {
   return *c;
 }
 
-const char* kMatmulColumns = "#columns,m,k,n,dtype,arch,kernel,tile_m,tile_n,tile_k,waves,split_k";
+// The mark behind the columns numbers the set of variants an autotune chooses
+// among; raise it when a variant is added.
+const char* kMatmulColumns = "#columns,m,k,n,dtype,arch,kernel,tile_m,tile_n,tile_k,waves,split_k,variants:2";
+const char* kMatmulArch = "gfx950";
 
-// Parses rows into a table; false for a bad header.
-bool parseMatmul(const std::string& path, std::map<Key, TuneEntry>* table, std::vector<std::string>* foreign,
-                 bool* opened) {
+// Parses rows into a table; false for a bad header.  `implicit`: the file is
+// the working directory's (or the environment's), not one the program asked
+// for.  gfx950 rows of such a file that were written ("#columns") by a build
+// with another set of variants are dropped, so those shapes are timed again; a
+// file without a "#columns" line was made by hand and keeps its rows.
+bool parseMatmul(const std::string& path, bool implicit, std::map<Key, TuneEntry>* table,
+                 std::vector<std::string>* foreign, bool* opened) {
   bool header_ok = true;
   std::vector<std::vector<std::string>> rows;
-  *opened = readCacheFile(path, "matmul", &header_ok, &rows);
+  std::string columns;
+  *opened = readCacheFile(path, "matmul", &header_ok, &rows, &columns);
+  const bool stale = implicit && !columns.empty() && columns != kMatmulColumns;
   if (!*opened) {
     return true;
   }
@@ -150,6 +163,9 @@ bool parseMatmul(const std::string& path, std::map<Key, TuneEntry>* table, std::
   }
   for (const auto& c : rows) {
     if (c.size() == 11) {
+      if (stale && c[4] == kMatmulArch) {
+        continue;
+      }
       try {
         TuneEntry e;
         e.kernel = c[5];
@@ -202,7 +218,7 @@ void loadMatmulOnce(MatmulCache& c) {
   bool opened = false;
   std::map<Key, TuneEntry> t;
   std::vector<std::string> foreign;
-  if (parseMatmul(c.path, &t, &foreign, &opened)) {
+  if (parseMatmul(c.path, true, &t, &foreign, &opened)) {
     for (auto& kv : t) {
       c.table.insert(kv);  // entries recorded before the load win
     }
@@ -503,7 +519,7 @@ lcError_t lcHipTuneCacheLoad(const char* path) {
   std::map<Key, TuneEntry> t;
   std::vector<std::string> foreign;
   bool opened = false;
-  const bool ok = parseMatmul(path, &t, &foreign, &opened);
+  const bool ok = parseMatmul(path, false, &t, &foreign, &opened);
   MatmulCache& c = mm();
   std::lock_guard<std::mutex> lock(c.mu);
   if (!opened) {

@@ -110,6 +110,39 @@ def test_cache_foreign_header_clears(tmp_path):
     """, tmp_path)
 
 
+def test_matmul_rows_of_another_variant_set_are_timed_again(tmp_path):
+    """The working directory's cache file, when an earlier build's autotune wrote
+    it ("#columns" without this build's variant-set mark): its gfx950 rows are
+    dropped, since they were chosen among fewer variants; rows of another arch
+    and the reference's stay.  Files that this build wrote, that were made by
+    hand, or that the program loads itself keep every row."""
+    cache = tmp_path / ".lightning_core_matmul_tune_cache.csv"
+    out = tmp_path / "out.csv"
+    old = "#columns,m,k,n,dtype,arch,kernel,tile_m,tile_n,tile_k,waves,split_k"
+    rows = ["1024,1024,1024,0,gfx950,f32_dp_64x64x64,64,64,64,8,2",
+            "300,400,500,1,gfx950,half_mid_128x128,128,128,64,4,1",
+            "1024,1024,1024,0,gfx942,f32_dp_64x64x64,64,64,64,8,2",
+            "64,64,64,16,1,0"]
+
+    def saved(load=None):
+        _run(f"""
+            import lightning_core as lc
+            {f"lc.tune_cache_load({str(load)!r})" if load else ""}
+            lc.tune_cache_save({str(out)!r})
+        """, tmp_path)
+        lines = _lines(out)
+        return lines[1], sorted(lines[2:])
+
+    cache.write_text("\n".join(["#lc_tune_cache,matmul,2", old] + rows) + "\n", encoding="utf-8")
+    columns, kept = saved()
+    assert columns.startswith(old) and columns != old
+    assert kept == sorted(rows[2:])
+    assert saved(load=cache)[1] == sorted(rows)
+    for header in ([columns], []):
+        cache.write_text("\n".join(["#lc_tune_cache,matmul,2"] + header + rows) + "\n", encoding="utf-8")
+        assert saved()[1] == sorted(rows)
+
+
 def test_attention_cache_seed_and_rows(tmp_path):
     seed = tmp_path / "attn_seed.csv"
     seed.write_text("#lc_tune_cache,attention,1\nfwd,8,8,0,0,0,0\n", encoding="utf-8")

@@ -41,6 +41,8 @@ constexpr std::size_t kMinChunk = std::size_t{256} << 10;
 //   down: wait for the slot's DMA, move the chunk out, enqueue the slot's next;
 //   up:   wait for the slot's last DMA (of this copy or an earlier one), move
 //         the chunk in, enqueue its DMA.
+// Waits on events spin, so the other threads join only once the stream has
+// reached the copy.
 struct Transfer {
   HipContext* ctx = nullptr;
   bool down = false;
@@ -49,6 +51,7 @@ struct Transfer {
   std::size_t bytes = 0, chunk = 0;
   int n = 0;
   int threads = 1;             // that share the slots: thread w has slots w, w + threads, ...
+  int first = 0, end = 0;      // the chunks they move; first is a multiple of kSlots
   std::atomic<int> error{0};   // first hipError_t; everyone stops
 
   std::size_t size(int i) const { return i + 1 < n ? chunk : bytes - static_cast<std::size_t>(i) * chunk; }
@@ -79,22 +82,33 @@ class Engine {
     while (t.chunk < kSlotBytes && t.chunk * 2 * kSlots <= bytes) {
       t.chunk *= 2;  // a ring's worth of chunks, or more
     }
-    t.n = static_cast<int>((bytes + t.chunk - 1) / t.chunk);
-    t.threads = helpers_ + 1;
+    t.n = t.end = static_cast<int>((bytes + t.chunk - 1) / t.chunk);
     if (down) {
       for (int i = 0; i < kSlots && i < t.n && !t.failed(); ++i) {
         enqueue(t, i);
       }
-      // The stream may have work before the copy: the helpers are woken only
-      // once the first chunk is here.
+      // The helpers are woken once the first chunk is here.
       const hipError_t e = t.failed() ? hipSuccess : hipEventSynchronize(events_[0]);
       if (e != hipSuccess) {
         t.fail(e);
       }
-      if (t.failed()) {
-        return static_cast<hipError_t>(t.error.load());
+    } else if (hipStreamQuery(ctx->stream) != hipSuccess) {
+      // The stream is busy: the caller fills the ring alone, and the helpers are
+      // woken once its first slot is free again.
+      (void)hipGetLastError();
+      t.end = kSlots < t.n ? kSlots : t.n;
+      work(t, 0);
+      t.first = t.end;
+      t.end = t.n;
+      const hipError_t e = t.failed() ? hipSuccess : hipEventSynchronize(events_[0]);
+      if (e != hipSuccess) {
+        t.fail(e);
       }
     }
+    if (t.failed()) {
+      return static_cast<hipError_t>(t.error.load());
+    }
+    t.threads = helpers_ + 1;
     {
       std::lock_guard<std::mutex> lock(mu_);
       current_ = &t;
@@ -159,8 +173,8 @@ class Engine {
   }
 
   void work(Transfer& t, int w) {
-    for (int first = 0; first < t.n; first += kSlots) {
-      for (int s = w; s < kSlots && first + s < t.n; s += t.threads) {
+    for (int first = t.first; first < t.end; first += kSlots) {
+      for (int s = w; s < kSlots && first + s < t.end; s += t.threads) {
         const int i = first + s;
         if (t.failed()) {
           return;

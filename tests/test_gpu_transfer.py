@@ -7,11 +7,12 @@ row above, a ring's worth and a remainder, and one with partly filled chunks.
 """
 import ctypes
 import threading
+import time
 
 import numpy as np
 import pytest
 
-from gpu_util import require_hip
+from gpu_util import note, require_hip
 
 pytestmark = pytest.mark.gpu
 
@@ -58,6 +59,40 @@ def test_two_threads_copy_at_once(lc):
     assert len(results) == 2
     for got, want in results.values():
         assert np.array_equal(got, want)
+
+
+def test_upload_behind_queued_work(lc):
+    """An upload that the stream reaches later arrives whole, and only the caller
+    waits for the queue: a waiting thread spins, so the processor time stays
+    below two cores (the caller's, and half again for the threads that copy once
+    the queue has drained; all four spinning would take four)."""
+    rng = np.random.default_rng(5)
+    n = 4096
+    busy = lc.MatMulResidentSession(n, n, n, "bf16")
+    a = rng.standard_normal((n, n), dtype=np.float32)
+    busy.start_into(a, a)
+    busy.sync_into()
+    rows = 2 * MIB + 5  # 32 MB and a remainder
+    x = rng.integers(-8, 9, (rows, 4)).astype(np.float32)
+    w = rng.integers(-8, 9, (4, 4)).astype(np.float32)
+    s = lc.MatMulResidentSession(rows, 4, 4, "f32")
+    s.start_into(x, w)
+    out = np.empty((rows, 4), np.float32)
+    s.finish_into(out=out)
+    for _ in range(2):
+        x = rng.integers(-8, 9, (rows, 4)).astype(np.float32)
+        for _ in range(250):  # below the count at which a launch waits for the queue
+            busy.run_into()
+        wall, cpu = time.perf_counter(), time.process_time()
+        s.start_into(x, w)
+        wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+        note(f"[transfer] upload behind queued work: {wall * 1e3:.1f} ms, {cpu / wall:.2f} cores")
+        assert wall > 0.01  # the queue was there
+        assert cpu < 2 * wall
+        s.finish_into(out=out)
+        assert np.array_equal(out, sum(x[:, i : i + 1] * w[i : i + 1] for i in range(4)))
+    s.close()
+    busy.close()
 
 
 def test_pinned_result_buffer(lc):

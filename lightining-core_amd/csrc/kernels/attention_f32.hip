@@ -236,8 +236,18 @@ __global__ __launch_bounds__(256 * KG, DK <= 2 ? 2 : 1) void attn_fwd_f32_split_
   };
 
   if (*in.guard == in.epoch) {
-    // the fp32 operands, straight from memory
+    // The fp32 operands, straight from memory, each tile's K and Q rows as
+    // float4 (one launch: the host then knows and takes attn_fwd_f32_kernel).
+    // Bound: the latency of those loads, few waves in flight.  Measured against
+    // that kernel (with its combine / with the planes and the combine here, us):
+    // 1x1024x128 43.6 -> 45.0, 1x600x128 39.1 -> 37.4, 8x1000x64 causal 71 -> 46,
+    // 48x2048x64 865 -> 693, 64x512x128 321 -> 144, 16x1500x96 causal 324 -> 262.
     const size_t base = static_cast<size_t>(head) * S * D;
+    const float* qp[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      qp[c] = in.q + base + static_cast<size_t>(min(q0 + 16 * c + lr, S - 1)) * D + 8 * lq;
+    }
     for (int t = t0 + kg; t <= last_tile; t += KG) {
       const int j0 = t * 32;
       floatx4 st[2][2];
@@ -246,16 +256,47 @@ __global__ __launch_bounds__(256 * KG, DK <= 2 ? 2 : 1) void attn_fwd_f32_split_
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
           st[r][c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-          const float* kp = in.k + base + static_cast<size_t>(min(j0 + 16 * r + lr, S - 1)) * D + 8 * lq;
-          const float* qp = in.q + base + static_cast<size_t>(min(q0 + 16 * c + lr, S - 1)) * D + 8 * lq;
-          for (int s = 0; s < D; s += 32) {
+        }
+      }
+      const float* kp[2];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              st[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(kp[s + e], qp[s + e], st[r][c], 0, 0, 0);
+      for (int r = 0; r < 2; ++r) {
+        kp[r] = in.k + base + static_cast<size_t>(min(j0 + 16 * r + lr, S - 1)) * D + 8 * lq;
+      }
+#pragma unroll
+      for (int s = 0; s < DK; ++s) {
+        floatx4 kf[2][2], qf[2][2];  // rows, halves of eight values
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            kf[r][h] = *reinterpret_cast<const floatx4*>(kp[r] + 32 * s + 4 * h);
+            qf[r][h] = *reinterpret_cast<const floatx4*>(qp[r] + 32 * s + 4 * h);
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              st[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[r][e / 4][e % 4], qf[c][e / 4][e % 4], st[r][c], 0, 0, 0);
             }
           }
         }
       }
+      // V's loads of two bands go out before the probabilities are needed
+      const float* vp = in.v + base + lr;
+      auto band = [&](int d, float (&x)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int key = j0 + 16 * (e / 4) + 4 * lq + e % 4;
+          x[e] = key < S ? vp[static_cast<size_t>(key) * D + 16 * d] : 0.0f;
+        }
+      };
+      float vx[2][8];
+      band(0, vx[0]);
+      band(1, vx[1]);
       float mt[2];
       probabilities(st, mt, true, j0);
       rescale(st, mt);
@@ -263,12 +304,13 @@ __global__ __launch_bounds__(256 * KG, DK <= 2 ? 2 : 1) void attn_fwd_f32_split_
       for (int d = 0; d < DB; ++d) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          const int key = j0 + 16 * (e / 4) + 4 * lq + e % 4;
-          const float a = key < S ? in.v[base + static_cast<size_t>(key) * D + 16 * d + lr] : 0.0f;
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
-            o[c][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, st[e / 4][c][e % 4], o[c][d], 0, 0, 0);
+            o[c][d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vx[d % 2][e], st[e / 4][c][e % 4], o[c][d], 0, 0, 0);
           }
+        }
+        if (d + 2 < DB) {
+          band(d + 2, vx[d % 2]);
         }
       }
     }

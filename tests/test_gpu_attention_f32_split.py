@@ -81,7 +81,7 @@ def test_split_forward_resident_and_postprocess(lc):
     sess.close()
 
 
-@pytest.mark.parametrize("b,h,s,d", [(1, 9, 520, 64), (1, 2, 200, 128)])
+@pytest.mark.parametrize("b,h,s,d", [(1, 9, 520, 64), (1, 2, 200, 128), (2, 40, 127, 32), (1, 3, 300, 96)])
 @pytest.mark.parametrize("what", ["nan", "inf", "tiny", "huge"])
 def test_operands_outside_the_split(lc, b, h, s, d, what):
     q, k, v = _inputs((b, h, s, d))

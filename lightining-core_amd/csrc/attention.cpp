@@ -339,7 +339,8 @@ namespace {
 // small enough for the 16-query kernel (4 heads of S = 256: 7.5 against 12.6
 // us), nor one head up to S = 2048 at D <= 64, where that kernel and the
 // 32-query kernel's key splits are as fast (S = 2048: 23.2 against 23.4 us).
-// The planes take 4.5 times a tensor's fp32 bytes: at most an eighth of memory.
+// The planes take 4.5 times a tensor's fp32 bytes: at most an eighth of memory,
+// and they are given up when another allocation needs it.
 bool splitServes(const HipContext* ctx, const AttnShape& sh) {
   const int S = static_cast<int>(sh.seq_len);
   const int D = static_cast<int>(sh.head_dim);
@@ -361,10 +362,19 @@ bool ensurePlanes(HipContext* ctx, AttnResident& res, const AttnShape& sh, hipEr
   const int D = static_cast<int>(sh.head_dim);
   const int bh = static_cast<int>(sh.bh());
   *e = hipSuccess;
+  const std::size_t bytes = kern::attentionF32PlanesHalves(bh, S, D) * sizeof(uint16_t);
+  if (res.planes.size() < bytes) {
+    res.has_planes = false;  // never made, too small, or freed for another allocation
+  }
   if (!res.has_planes) {
-    if (res.planes.ensure(kern::attentionF32PlanesHalves(bh, S, D) * sizeof(uint16_t)) != Status::kSuccess) {
+    if (res.planes_denied == ctx->frees) {
       return false;
     }
+    if (res.planes.ensureSpare(ctx, bytes) != Status::kSuccess) {
+      res.planes_denied = ctx->frees;
+      return false;
+    }
+    res.planes_denied = 0;
     const GuardArgs g = beginGuard(ctx, &res.guard_slot, 0);
     res.epoch = g.epoch;
     if (g.epoch == 0) {
@@ -407,6 +417,7 @@ Status attentionForwardResident(HipContext* ctx, AttnResident& res, const AttnSh
   }
   if (policy.upload_q || policy.upload_k || policy.upload_v) {
     res.has_planes = false;
+    res.planes_denied = 0;
   }
   if ((!policy.upload_q && !res.has_q) || (!policy.upload_k && !res.has_k) || (!policy.upload_v && !res.has_v)) {
     return fail(Status::kInvalidValue, "attention: no resident input for a tensor the policy does not upload");
@@ -438,13 +449,14 @@ Status attentionForwardResident(HipContext* ctx, AttnResident& res, const AttnSh
   const std::size_t hint = sh.seq_len * sh.seq_len * sh.head_dim;
   int splits = 0;  // batched fp32 heads keep the heuristic (the cache keys one head)
   hipError_t planes_error = hipSuccess;
-  const bool planes = repeat > 0 && splitServes(ctx, sh) && ensurePlanes(ctx, res, sh, &planes_error);
+  const int cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
+  bool planes = repeat > 0 && splitServes(ctx, sh);
+  if (planes) {  // the workspace first: an allocation may free planes
+    LC_TRY(ensureSplitWs(res, kern::attentionF32SplitWorkFloats(bh, S, D, cus)));
+    planes = ensurePlanes(ctx, res, sh, &planes_error);
+  }
   if (planes_error != hipSuccess) {
     return failHip(planes_error, "attention operand planes");
-  }
-  const int cus = ctx->props.multiProcessorCount > 0 ? ctx->props.multiProcessorCount : 256;
-  if (planes) {
-    LC_TRY(ensureSplitWs(res, kern::attentionF32SplitWorkFloats(bh, S, D, cus)));
   }
   if (!half && !planes && bh == 1 && repeat > 0) {
     LC_TRY(forwardSplits(ctx, res, sh, policy, &splits));
@@ -847,6 +859,7 @@ lcError_t lcAttentionSessionDestroy(lcAttentionSession* session) {
     std::lock_guard<std::recursive_mutex> lock(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);  // no kernel may still use the buffers
     releaseGuard(ctx, &session->res.guard_slot);
+    dropSpare(ctx, &session->res.planes);
     delete session;
   } else {
     delete session;

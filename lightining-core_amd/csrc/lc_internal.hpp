@@ -8,6 +8,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <mutex>
@@ -73,6 +74,7 @@ int encodeDispatch(Device requested, Device selected, bool fallback);
 // Device allocation that grows (1.5x, like the reference's Metal buffers,
 // src/attention_metal.mm:150-164) and never shrinks.  Contents are not kept
 // across growth.  Freed by reset() or the destructor.
+struct HipContext;
 class DeviceBuffer {
  public:
   DeviceBuffer() = default;
@@ -80,6 +82,9 @@ class DeviceBuffer {
   DeviceBuffer& operator=(const DeviceBuffer&) = delete;
   ~DeviceBuffer() { reset(); }
   Status ensure(std::size_t bytes, bool zero = false);
+  // The same for a spare (HipContext::spares): the exact size, and a failure
+  // frees no other spare.  dropSpare before the buffer is destroyed.
+  Status ensureSpare(HipContext* ctx, std::size_t bytes);
   void reset();
   void* get() const { return ptr_; }
   template <typename T>
@@ -150,6 +155,13 @@ struct HipContext {
   DeviceBuffer guard_words;
   PinnedBuffer guard_host;
   std::vector<int> guard_free;
+  // Spare buffers: contents that can be made again (the bf16 planes of fp32
+  // operands).  They are freed when another allocation fails, so a spare's owner
+  // looks at its size before each use.
+  std::vector<DeviceBuffer*> spares;
+  // Counts the library's frees of device memory: a spare that could not be had
+  // is asked for again after an upload or a free.
+  std::atomic<std::size_t> frees{1};
   int guard_epoch = 0;
   // Enqueue-only launches since the stream was last synchronised, per op
   // family (noteEnqueued; syncStream resets both).
@@ -166,6 +178,9 @@ struct HipContext {
 };
 
 bool hipAvailable();
+// Frees every spare (ctx->mu held); whether there was one.
+bool freeSpares(HipContext* ctx);
+void dropSpare(HipContext* ctx, DeviceBuffer* b);
 // Returns the context, or nullptr with the status set (kNotSupported when no
 // gfx950 device is visible).
 HipContext* hipContext(Status* st);

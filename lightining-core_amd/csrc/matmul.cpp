@@ -69,6 +69,7 @@ GuardArgs beginUpload(HipContext* ctx, MatMulResident& r, int which) {
   const GuardArgs g = beginGuard(ctx, &r.guard_slot, which);
   (which == 0 ? r.epoch_a : r.epoch_b) = g.epoch;
   (which == 0 ? r.has_planes_a : r.has_planes_b) = false;
+  r.planes_denied = 0;
   return g;
 }
 
@@ -259,7 +260,8 @@ int cuCount(const HipContext* ctx) {
 
 // The split GEMM keeps 6 bytes more per operand value; past an eighth of the
 // device's memory, or past the kernels' 32-bit offsets along k (160 bytes a k),
-// the fp32 kernels run instead.
+// the fp32 kernels run instead.  The planes are given up when another
+// allocation needs their memory.
 bool splitFits(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t n) {
   const std::size_t kp = roundUp(k, kern::kF32GemmBK);
   const std::size_t rows = roundUp(m, kern::kF32GemmBM) + roundUp(n, kern::kF32GemmBN);
@@ -288,11 +290,16 @@ bool launchSplitGemm(HipContext* ctx, MatMulResident& r, kern::GemmF32Variant va
   const std::size_t na = 3 * static_cast<std::size_t>(mp) * kp;
   const std::size_t nb = 3 * static_cast<std::size_t>(np) * kp;
   if (r.planes.size() < (na + nb) * sizeof(uint16_t)) {
-    r.has_planes_a = r.has_planes_b = false;  // growth drops the contents
+    r.has_planes_a = r.has_planes_b = false;  // never made, too small, or freed for another allocation
   }
-  if (r.planes.ensure((na + nb) * sizeof(uint16_t)) != Status::kSuccess) {
+  if (r.planes_denied == ctx->frees) {
     return false;
   }
+  if (r.planes.ensureSpare(ctx, (na + nb) * sizeof(uint16_t)) != Status::kSuccess) {
+    r.planes_denied = ctx->frees;
+    return false;
+  }
+  r.planes_denied = 0;
   const kern::SplitOperandF32 a{r.a.as<float>(), kp, mp / 16, r.planes.as<uint16_t>()};
   const kern::SplitOperandF32 b{r.b.as<float>(), np, np / 16, r.planes.as<uint16_t>() + na};
   if (!r.has_planes_a || !r.has_planes_b) {
@@ -828,6 +835,7 @@ lcError_t lcMatMulResidentSessionDestroy(lcMatMulResidentSession* s) {
     std::lock_guard<std::recursive_mutex> lock(ctx->mu);
     (void)hipStreamSynchronize(ctx->stream);
     releaseGuard(ctx, &s->res.guard_slot);
+    dropSpare(ctx, &s->res.planes);
   }
   delete s;
   return LC_SUCCESS;

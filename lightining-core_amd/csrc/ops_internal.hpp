@@ -52,8 +52,9 @@ struct AttnResident {
   DeviceBuffer split_ws;   // partials of the fp32 forward's key splits
   // fp32: the bf16 parts of q, k and v (kern::AttnPlanesF32), made when the
   // forward first needs them after one of the three has changed.
-  DeviceBuffer planes;
+  DeviceBuffer planes;  // a spare
   bool has_planes = false;
+  std::size_t planes_denied = 0;  // HipContext::frees when there was no memory for them (0: there was)
   int guard_slot = -1;
   int epoch = 0;
   bool has_q = false, has_k = false, has_v = false, has_out = false, has_target = false;
@@ -93,8 +94,9 @@ struct MatMulResident {
   bool once_tuned = false;
   // fp32: the bf16 parts of A, then of B (kern::SplitOperandF32), made when a
   // split GEMM first needs them after an upload.
-  DeviceBuffer planes;
+  DeviceBuffer planes;  // a spare
   bool has_planes_a = false, has_planes_b = false;
+  std::size_t planes_denied = 0;  // HipContext::frees when there was no memory for them (0: there was)
   // fp32: this resident's guard slot (-1: none) and the epochs of the
   // operands' last uploads (0: not guarded).
   int guard_slot = -1;

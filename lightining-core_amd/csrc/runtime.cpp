@@ -11,6 +11,7 @@
 // HIP replaces CUDA/Metal: malloc/free/memcpy map to hipMalloc/hipFree/
 // hipMemcpy, deviceSynchronize drains the backend stream, the memory model is
 // native-device, and the preferred device is hip when a gfx950 is visible.
+#include <algorithm>
 #include <atomic>
 #include <chrono>
 #include <cstdarg>
@@ -169,6 +170,36 @@ HipContext* hipContext(Status* st) {
 
 bool hipAvailable() { return hipContext(nullptr) != nullptr; }
 
+bool freeSpares(HipContext* ctx) {
+  bool any = false;
+  for (DeviceBuffer* b : ctx->spares) {
+    any = any || b->get() != nullptr;
+    b->reset();  // hipFree waits for kernels that still read it
+  }
+  return any;
+}
+
+Status DeviceBuffer::ensureSpare(HipContext* ctx, std::size_t bytes) {
+  if (bytes <= bytes_ && ptr_ != nullptr) {
+    return Status::kSuccess;
+  }
+  reset();
+  const hipError_t e = hipMalloc(&ptr_, bytes);
+  if (e != hipSuccess) {
+    ptr_ = nullptr;
+    return failHip(e, "hipMalloc");
+  }
+  bytes_ = bytes;
+  if (std::find(ctx->spares.begin(), ctx->spares.end(), this) == ctx->spares.end()) {
+    ctx->spares.push_back(this);
+  }
+  return Status::kSuccess;
+}
+
+void dropSpare(HipContext* ctx, DeviceBuffer* b) {
+  ctx->spares.erase(std::remove(ctx->spares.begin(), ctx->spares.end(), b), ctx->spares.end());
+}
+
 Status DeviceBuffer::ensure(std::size_t bytes, bool zero) {
   if (bytes <= bytes_ && ptr_ != nullptr) {
     return Status::kSuccess;
@@ -183,8 +214,12 @@ Status DeviceBuffer::ensure(std::size_t bytes, bool zero) {
   hipError_t e = hipMalloc(&p, want);
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    // retry with the exact size before giving up
+    // retry with the exact size, then without the spare buffers, before giving up
     e = hipMalloc(&p, bytes);
+    if (e != hipSuccess && g_ctx != nullptr && freeSpares(g_ctx)) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, bytes);
+    }
     if (e != hipSuccess) {
       return failHip(e, "hipMalloc");
     }
@@ -209,6 +244,9 @@ Status DeviceBuffer::ensure(std::size_t bytes, bool zero) {
 void DeviceBuffer::reset() {
   if (ptr_ != nullptr) {
     (void)hipFree(ptr_);
+    if (g_ctx != nullptr) {
+      ++g_ctx->frees;
+    }
   }
   ptr_ = nullptr;
   bytes_ = 0;
@@ -402,6 +440,13 @@ Status mallocDevice(void** ptr, std::size_t size_bytes) {
     *ptr = nullptr;
   } else {
     hipError_t e = hipMalloc(ptr, size_bytes);
+    if (e != hipSuccess) {
+      std::lock_guard<std::recursive_mutex> lock(ctx->mu);
+      if (freeSpares(ctx)) {
+        (void)hipGetLastError();
+        e = hipMalloc(ptr, size_bytes);
+      }
+    }
     st = (e == hipSuccess) ? Status::kSuccess : failHip(e, "hipMalloc");
   }
   traceRecord(TraceEventType::kMallocDevice, st, size_bytes);
@@ -414,6 +459,7 @@ Status freeDevice(void* ptr) {
     HipContext* ctx = hipContext(&st);
     if (ctx != nullptr) {
       hipError_t e = hipFree(ptr);
+      ++ctx->frees;
       st = (e == hipSuccess) ? Status::kSuccess : failHip(e, "hipFree");
     }
   }

@@ -390,8 +390,9 @@ lcError_t lcMatMulResidentSessionRunBatchSyncCachedNoDownload(lcMatMulResidentSe
  * single kernel).  TimeLaunches: `count` launch-only GEMMs on the resident
  * inputs, back to back on the backend stream with a hipEvent pair around each
  * launch, then a sync; ms_out[i] = launch i's event-measured duration.
- * KernelName: "<tune-cache variant> <kernel function>" of the GEMM the
- * session's shape runs (e.g. "half_w4h_256x256 gemm_half_tn_w4h_kernel"). */
+ * KernelName: "<tune-cache variant> <kernel function>" of the GEMM that the
+ * session's shape and resident operands run (e.g. "half_w4h_256x256
+ * gemm_half_tn_w4h_kernel"). */
 lcError_t lcMatMulResidentSessionTimeLaunches(lcMatMulResidentSession* s, size_t count, float* ms_out);
 lcError_t lcMatMulResidentSessionKernelName(lcMatMulResidentSession* s, char* buf, size_t cap);
 

@@ -947,9 +947,19 @@ lcError_t lcMatMulResidentSessionKernelName(lcMatMulResidentSession* s, char* bu
   }
   std::lock_guard<std::recursive_mutex> lock(ctx->mu);
   const bool half = isHalf(s->dtype);
-  int v = s->res.tuned ? s->res.variant : 0;
+  const MatMulResident& r = s->res;
+  int v = r.tuned ? r.variant : 0;
   if (v == 0) {
     v = half ? defaultHalfVariant(ctx, s->m, s->k, s->n) : defaultF32Variant(ctx, s->m, s->k, s->n);
+  }
+  // Operands the split GEMM does not take, planes past their limit or without
+  // memory: the fp32 instruction's variant runs.
+  if (!half && isSplit(v) &&
+      (!splitFits(ctx, s->m, s->k, s->n) || r.planes_denied == ctx->frees || (r.has_a && r.has_b && knownUnsafe(ctx, r)))) {
+    v = r.once;
+    if (v == 0) {
+      v = static_cast<int>(kern::gemmF32Choose(static_cast<int>(s->m), static_cast<int>(s->n), cuCount(ctx)));
+    }
   }
   std::string text;
   for (const VariantInfo& info : variants(half)) {

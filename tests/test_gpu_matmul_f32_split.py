@@ -203,3 +203,24 @@ def test_unfit_operands_settle_no_split_choice(lc, tmp_path):
         assert bar and not resident and "split" not in once
     name, kernel = rows[2]
     assert name.partition("|")[2] == kernel and "split" in kernel
+
+
+def test_kernel_name_follows_the_operands(lc):
+    """kernel_name() is the GEMM that runs: with operands the split GEMM does not
+    take it names the fp32 instruction's kernel, and the shape's own again after
+    the next fit upload."""
+    rng = np.random.default_rng(10)
+    m, k, n = 640, 2048, 640
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, n), dtype=np.float32)
+    bad = a.copy()
+    bad[3, 5] = np.inf
+    s = lc.MatMulResidentSession(m, k, n)
+    names = {True: set(), False: set()}
+    for x in (a, bad, a, bad):
+        s.start_into(x, b)
+        s.finish_into()
+        names[x is a].add(s.kernel_name().split()[0])
+    s.close()
+    assert len(names[True]) == 1 and "split" in names[True].pop()
+    assert not any("split" in x for x in names[False])

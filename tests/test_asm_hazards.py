@@ -259,3 +259,21 @@ def test_built_kernels_have_no_lds_dma_hazards(tmp_path):
                 spills.append(f"{os.path.basename(out)}: {name} private segment {m.group(1) if m else '?'} bytes")
     assert kernels > 0, "no kernel descriptors found"
     assert not spills, "\n".join(spills[:20])
+
+
+@pytest.mark.skipif(not shutil.which(HIPCC) and not os.path.exists(HIPCC), reason="hipcc not available")
+def test_row_sums_stay_between_the_score_mfmas(tmp_path):
+    """16-bit attention, D = 128: a group's row sum (one packed dot) is issued
+    behind the group's MFMA, which hides it; the compiler can move all of a
+    tile's sums to its end, where nothing does."""
+    text = open(_compile_asm(os.path.join(CSRC, "kernels", "attention.hip"), str(tmp_path))).read()
+    longest = {}
+    for name, body in re.findall(r"^(_Z\S*attn_fwd_half_\S*Li128E\S*):(.*?)\.end_amdhsa_kernel", text, re.S | re.M):
+        run = longest[name] = 0
+        for t in _instructions(body):
+            if t.startswith("v_dot2"):
+                run += 1
+                longest[name] = max(longest[name], run)
+            elif t.startswith("v_mfma"):
+                run = 0
+    assert len(longest) == 6 and all(1 <= n <= 2 for n in longest.values()), longest

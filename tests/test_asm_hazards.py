@@ -235,12 +235,19 @@ def test_scan_catches_a_sign_extended_readfirstlane_base():
     assert scan(fixed) == []
 
 
-@pytest.mark.skipif(not shutil.which(HIPCC) and not os.path.exists(HIPCC), reason="hipcc not available")
-def test_built_kernels_have_no_lds_dma_hazards(tmp_path):
+@pytest.fixture(scope="module")
+def outs(tmp_path_factory):
+    """The assembly of every kernel source, compiled once."""
+    if not shutil.which(HIPCC) and not os.path.exists(HIPCC):
+        pytest.skip("hipcc not available")
     srcs = sorted(glob.glob(os.path.join(CSRC, "kernels", "*.hip")))
     assert srcs
+    out_dir = str(tmp_path_factory.mktemp("asm"))
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(4, len(srcs))) as ex:
-        outs = list(ex.map(lambda s: _compile_asm(s, str(tmp_path)), srcs))
+        return list(ex.map(lambda s: _compile_asm(s, out_dir), srcs))
+
+
+def test_built_kernels_have_no_lds_dma_hazards(outs):
     loads = 0
     problems = []
     for out in outs:
@@ -261,12 +268,11 @@ def test_built_kernels_have_no_lds_dma_hazards(tmp_path):
     assert not spills, "\n".join(spills[:20])
 
 
-@pytest.mark.skipif(not shutil.which(HIPCC) and not os.path.exists(HIPCC), reason="hipcc not available")
-def test_row_sums_stay_between_the_score_mfmas(tmp_path):
+def test_row_sums_stay_between_the_score_mfmas(outs):
     """16-bit attention, D = 128: a group's row sum (one packed dot) is issued
     behind the group's MFMA, which hides it; the compiler can move all of a
     tile's sums to its end, where nothing does."""
-    text = open(_compile_asm(os.path.join(CSRC, "kernels", "attention.hip"), str(tmp_path))).read()
+    text = open(next(o for o in outs if os.path.basename(o) == "attention.hip.s")).read()
     longest = {}
     for name, body in re.findall(r"^(_Z\S*attn_fwd_half_\S*Li128E\S*):(.*?)\.end_amdhsa_kernel", text, re.S | re.M):
         run = longest[name] = 0

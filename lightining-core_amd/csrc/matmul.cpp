@@ -429,14 +429,24 @@ int defaultF32Variant(const HipContext* ctx, std::size_t m, std::size_t k, std::
 }
 
 // 16 bits: the skinny kernel up to 16 rows, 256x256 tiles while there is one
-// per CU, else the smaller tiles of gemm_half.hip (within its 32-bit offsets).
+// per CU, else the smaller tiles of gemm_half.hip (within its 32-bit offsets)
+// unless the product is mostly stores: few k steps, or rows of C that no 16-byte
+// store fits, in more than a few tiles.  There the register-staged kernels,
+// several workgroups a CU, hide the stores (us, them / the ring tiles):
+// 7044x157x1759 19.7 / 44.7, 1360x581x6939 29.0 / 42.9, 6208x64x832 9.4 / 12.5,
+// 2304x384x5760 24.9 / 29.1; past the lines 13568x384x704 21.8 / 22.6,
+// 1920x640x6656 34.1 / 37.5, 1500x3000x2000 39.6 / 22.9.  Over 440 shapes the rule's
+// choice is 0.5% behind the better of the two, 14% at worst.
 int defaultHalfVariant(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t n) {
   const int M = static_cast<int>(m);
   const int N = static_cast<int>(n);
   const kern::GemmHalfVariant v = kern::gemmHalfChoose(M, N);
   const int kp = static_cast<int>(roundUp(k, kern::kHalfGemmBK));
   if ((v == kern::GemmHalfVariant::kMid || v == kern::GemmHalfVariant::kSmall) && kern::gemmHalfR4Fits(kp, kp)) {
-    return static_cast<int>(kern::gemmHalfR4Choose(M, N, kp, cuCount(ctx)));
+    const bool stores = ((m + 127) / 128) * ((n + 127) / 128) >= 64 && kp <= (n % 4 == 0 ? 384 : 1280);
+    if (!stores) {
+      return static_cast<int>(kern::gemmHalfR4Choose(M, N, kp, cuCount(ctx)));
+    }
   }
   return static_cast<int>(v);
 }
@@ -541,12 +551,16 @@ Status settleVariant(HipContext* ctx, MatMulResident& r) {
         }
       }
     }
-  } else if (r.m > 16 && kern::gemmHalfR4Fits(roundUp(r.k, kern::kHalfGemmBK), roundUp(r.k, kern::kHalfGemmBK))) {
-    // The other kernels were slower than one of these at every shape tried;
-    // they stay for a tune cache or CJ_HIP_GEMM_TILE that names them.
-    cands = {static_cast<int>(kern::GemmHalfVariant::kW4H)};
+  } else if (r.m > 16) {
+    // w4, w4d, big8 and big4 were never more than 3% ahead of all of these over
+    // 440 shapes (17-16384 x 64-8192 x 64-8192); they stay for a tune cache or
+    // CJ_HIP_GEMM_TILE that names them.
+    cands = {static_cast<int>(kern::GemmHalfVariant::kW4H), static_cast<int>(kern::GemmHalfVariant::kW4R),
+             static_cast<int>(kern::GemmHalfVariant::kLds), static_cast<int>(kern::GemmHalfVariant::kMid),
+             static_cast<int>(kern::GemmHalfVariant::kSmall)};
+    const long long k_pad = static_cast<long long>(roundUp(r.k, kern::kHalfGemmBK));
     for (const VariantInfo& v : kHalfVariants) {
-      if (kern::isR4(static_cast<kern::GemmHalfVariant>(v.variant))) {
+      if (kern::isR4(static_cast<kern::GemmHalfVariant>(v.variant)) && kern::gemmHalfR4Fits(k_pad, k_pad)) {
         cands.push_back(v.variant);
       }
     }

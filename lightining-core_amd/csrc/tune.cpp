@@ -140,7 +140,7 @@ MatmulCache& mm() {
 
 // The mark behind the columns numbers the set of variants an autotune chooses
 // among; raise it when a variant is added.
-const char* kMatmulColumns = "#columns,m,k,n,dtype,arch,kernel,tile_m,tile_n,tile_k,waves,split_k,variants:2";
+const char* kMatmulColumns = "#columns,m,k,n,dtype,arch,kernel,tile_m,tile_n,tile_k,waves,split_k,variants:3";
 const char* kMatmulArch = "gfx950";
 
 // Parses rows into a table; false for a bad header.  `implicit`: the file is

@@ -72,3 +72,39 @@ def test_tiles_match_the_256_tile_bitwise(lc, tmp_path, dtype):
     for m, k, n, share in worst:
         note(f"[parity] {dtype} {m}x{k}x{n}: {float(share):.3f} of the bound")
         assert float(share) <= 1.0
+
+
+# More than 64 tiles of 128 x 128, few k steps or columns that no 16-byte store fits: the
+# register-staged kernels take about half of the ring tiles' time there.
+STORES = [(7044, 157, 1759), (3030, 91, 2554), (2034, 260, 6795)]
+# Long k: the ring tiles take about half of the others' time.
+LONG = [(1500, 3000, 2000), (378, 7510, 2692)]
+
+
+@pytest.mark.parametrize("tuned", ["1", "0"])
+def test_products_that_are_mostly_stores_keep_the_staged_kernels(lc, tmp_path, tuned):
+    """Both the timed choice and the heuristic's; results against float64 as above."""
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "lightining-core_amd"), CJ_MATMUL_AUTOTUNE=tuned)
+    r = subprocess.run([sys.executable, "-u", "-c", textwrap.dedent(f"""
+        import numpy as np
+        import lightning_core as lc
+        from lightning_core import synth
+        for m, k, n in {STORES + LONG!r}:
+            print("[case]", m, k, n, flush=True)
+            a, b = synth.normal((m, k), stream=53), synth.normal((k, n), stream=54)
+            s = lc.MatMulResidentSession(m, k, n, compute_dtype="bf16")
+            s.start_into(a, b)
+            name = s.kernel_name().split()[0]
+            c = s.finish_into().reshape(m, n)[-130:]
+            s.close()
+            a, b = (synth.round_to(x, "bf16").astype(np.float64) for x in (a[-130:], b))
+            bound = (k / 32 + 8) * 2.0 ** -22 * (np.abs(a) @ np.abs(b))
+            print("NAME", m, k, n, name, float((np.abs(c - a @ b) / bound).max()), flush=True)
+    """)], cwd=tmp_path, env=env, capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
+    names = [line.split()[1:] for line in r.stdout.splitlines() if line.startswith("NAME")]
+    assert len(names) == len(STORES + LONG)
+    for m, k, n, name, share in names:
+        note(f"[tune] {m}x{k}x{n}: {name}, {float(share):.3f} of the bound")
+        assert float(share) <= 1.0
+        assert ("_r4_" in name) == ((int(m), int(k), int(n)) in LONG)

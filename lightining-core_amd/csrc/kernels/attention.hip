@@ -2217,27 +2217,42 @@ hipError_t mseLossF32(const float* out, const float* target, size_t n, float nor
 }
 
 // How many waves share a query block's keys (attn_fwd_half_keys_kernel), or 1
-// for attn_fwd_half_kernel.  With W 32-query blocks in all, four waves a block
-// win while the blocks fit the chip at once (one per CU at D = 128, two at
-// D = 64 run slower, so up to 1.5 per CU), two waves until the K and V^T tiles
-// that every 32 queries load again cost more than the shorter chain saves;
-// causal blocks average half of the tiles and gain for longer.  Measured at the
-// lines (us: whole blocks of 128 / four / two waves; b x h x S x D):
-//   D 64   1x12x700 12.7/9.3/10.9  4x12x196 7.4/7.1/7.1  1x12x1400 21.2/19.8/18.2
-//          4x12x350 9.3/12.0/9.2   2x12x1400 29.2/30.3/29.9
-//   causal 1x12x1400 21.4/11.8/13.8  4x12x350 9.4/9.4/8.2  2x12x1400 22.4/20.6/18.9
-//          4x16x700 15.0/20.3/16.6
-//   D 128  1x4x1400 29.1/14.6/18.2  2x12x350 12.8/16.5/12.4  1x4x2800 52.1/37.8/40.4
-//          4x16x196 11.0/14.7/10.8  2x12x700 18.8/27.8/25.4
-//   causal 1x12x700 17.4/11.9/13.0  4x16x196 10.6/12.5/9.4  4x12x350 13.3/18.9/15.0
-//          2x12x700 17.9/20.8/15.9  2x12x1400 32.4/42.3/34.9
+// for attn_fwd_half_kernel.  Four waves win while the 32-query blocks fit the
+// chip at once (one per CU at D = 128, two at D = 64, as LDS allows; more where
+// long causal blocks average half of their tiles); two waves until the K and V^T
+// tiles that every 32 queries load again cost more than the shorter chain saves,
+// which takes longer the more tiles a block has.  A single tile (S <= 64) has
+// nothing to share; up to 32 queries, where the 128-query kernel leaves three
+// waves idle, two waves win in the middle.
+// Lines fitted to 6800 shapes timed with one, two and four waves (S 16-4096, up
+// to 7.5 blocks per CU): the choice takes 0.2% more than the best on average and
+// over 5% more for 1.4% of the shapes (22% at worst).  At the lines (us,
+// whole blocks of 128 / four / two waves; heads x S x D):
+//   D 64   176x44 4.7/-/5.6  176x82 5.9/-/6.9  529x31 6.9/8.5/6.0
+//   causal 117x278 9.8/-/13.7  172x160 8.4/10.0/7.4  2x1896 26.1/10.3/15.3
+//   D 128  37x303 12.2/-/15.6  116x65 7.8/-/9.4  12x839 21.0/21.4/18.1
+//          508x32 9.5/12.2/8.5  causal 64x206 10.7/12.7/9.6
 static int half_key_shares(int bh, int S, int D, bool causal, int cus) {
   const long long blocks = static_cast<long long>(bh) * ((S + 31) / 32);
   const long long eighths = (blocks * 8 + cus - 1) / cus;  // blocks per CU, in eighths
-  if (D == 64) {
-    return eighths <= 12 ? 4 : eighths <= (causal ? 34 : 17) ? 2 : 1;
+  if (S <= 64) {
+    return S <= 32 && (D == 64 ? eighths > 12 : eighths > 8 && eighths <= 16) ? 2 : 1;
   }
-  return eighths <= 8 ? 4 : eighths <= (!causal ? 12 : S < 512 ? 14 : 17) ? 2 : 1;
+  // Most eighths for four waves and for two, by [D = 128][causal][64-key tiles:
+  // up to 2, 4, 8, 12, 16, 24, 32, more].
+  constexpr int kTiles[7] = {2, 4, 8, 12, 16, 24, 32};
+  constexpr int kLines[2][2][8][2] = {
+      {{{9, 9}, {16, 16}, {16, 16}, {16, 18}, {16, 32}, {16, 32}, {16, 32}, {16, 32}},
+       {{16, 16}, {16, 25}, {16, 23}, {16, 27}, {17, 36}, {20, 48}, {22, 49}, {32, 54}}},
+      {{{8, 8}, {8, 8}, {8, 8}, {8, 15}, {8, 16}, {8, 16}, {8, 16}, {8, 16}},
+       {{8, 8}, {8, 12}, {8, 16}, {9, 18}, {10, 21}, {13, 27}, {16, 30}, {16, 30}}}};
+  const int tiles = (S + 63) / 64;
+  int row = 0;
+  while (row < 7 && tiles > kTiles[row]) {
+    ++row;
+  }
+  const int (&line)[2] = kLines[D == 128][causal][row];
+  return eighths <= line[0] ? 4 : eighths <= line[1] ? 2 : 1;
 }
 
 hipError_t attentionHalf(const uint16_t* q, const uint16_t* k, const uint16_t* vt, float* out_f32,

@@ -417,15 +417,23 @@ Status timeVariants(HipContext* ctx, MatMulResident& r, const std::vector<int>& 
   return Status::kSuccess;
 }
 
-// fp32: the split GEMM where its planes fit, else whole tiles or stream-K.
+// fp32: the split GEMM where its planes fit, else whole tiles or stream-K, and
+// those as well for the shortest k, where loads and stores are all there is: one
+// 64-deep step in at most one 64x64 tile per CU, or up to three in more tiles
+// whose rows no 16-byte store fits (us, them / the split GEMM): 948x45x631 5.7 /
+// 6.9, 710x51x1918 8.3 / 11.6, 3144x74x1342 21.7 / 30.6; past the lines
+// 1024x32x2816 11.4 / 9.7, 2048x80x1056 14.5 / 13.3.
+// Over 500 shapes 0.2% behind the better of the two, 15% at worst.
 int defaultF32Variant(const HipContext* ctx, std::size_t m, std::size_t k, std::size_t n) {
   const int M = static_cast<int>(m);
   const int N = static_cast<int>(n);
-  if (!splitFits(ctx, m, k, n)) {
+  const std::size_t kp = roundUp(k, kern::kF32GemmBK);
+  const bool one_round = ((m + 63) / 64) * ((n + 63) / 64) <= static_cast<std::size_t>(cuCount(ctx));
+  const bool short_k = one_round ? kp <= 64 : n % 4 != 0 && kp <= 192;
+  if (short_k || !splitFits(ctx, m, k, n)) {
     return static_cast<int>(kern::gemmF32Choose(M, N, cuCount(ctx)));
   }
-  return static_cast<int>(
-      kern::gemmF32SplitChoose(M, N, static_cast<int>(roundUp(k, kern::kF32GemmBK)), cuCount(ctx)));
+  return static_cast<int>(kern::gemmF32SplitChoose(M, N, static_cast<int>(kp), cuCount(ctx)));
 }
 
 // 16 bits: the skinny kernel up to 16 rows, 256x256 tiles while there is one

@@ -224,3 +224,30 @@ def test_kernel_name_follows_the_operands(lc):
     s.close()
     assert len(names[True]) == 1 and "split" in names[True].pop()
     assert not any("split" in x for x in names[False])
+
+
+def test_heuristic_keeps_whole_tiles_for_the_shortest_k(lc, tmp_path):
+    """Without autotune: one k step in few tiles, or a few in many tiles with rows
+    that no 16-byte store fits, run the fp32 instruction's kernels; the split GEMM
+    begins past those lines."""
+    shapes = {(948, 45, 631): False, (64, 64, 64): False, (710, 51, 1918): False, (1500, 190, 1501): False,
+              (1500, 193, 1501): True, (1024, 32, 2816): True, (1024, 65, 1024): True, (1024, 1024, 1024): True}
+    out = _child(f"""
+        import os
+        os.environ["CJ_MATMUL_AUTOTUNE"] = "0"
+        import numpy as np
+        import lightning_core as lc
+        from lightning_core import synth
+        for m, k, n in {list(shapes)!r}:
+            a, b = synth.normal((m, k), stream=81), synth.normal((k, n), stream=82)
+            s = lc.MatMulResidentSession(m, k, n)
+            s.start_into(a, b)
+            c = s.finish_into().reshape(m, n)
+            print("NAME", m, k, n, s.kernel_name().split()[0], flush=True)
+            s.close()
+            a, b = a.astype(np.float64), b.astype(np.float64)
+            bound = (k + 16) * 2.0 ** -23 * (np.abs(a) @ np.abs(b))
+            assert (np.abs(c - a @ b) <= bound).all()
+    """, tmp_path)
+    names = [line.split()[1:] for line in out.splitlines() if line.startswith("NAME")]
+    assert [("split" in name) for *_, name in names] == list(shapes.values())

@@ -251,3 +251,32 @@ def test_heuristic_keeps_whole_tiles_for_the_shortest_k(lc, tmp_path):
     """, tmp_path)
     names = [line.split()[1:] for line in out.splitlines() if line.startswith("NAME")]
     assert [("split" in name) for *_, name in names] == list(shapes.values())
+
+
+def _exact64(x):
+    """fp32 to fp64 bit by bit: a library built with -ffast-math may have set this
+    process to read subnormal values as zeros."""
+    u = x.view(np.uint32)
+    exponent = ((u >> 23) & 255).astype(np.int64)
+    mantissa = (u & 0x7FFFFF).astype(np.float64) + np.where(exponent > 0, 2.0 ** 23, 0.0)
+    return np.where(u >> 31, -1.0, 1.0) * np.ldexp(mantissa, np.maximum(exponent, 1) - 150)
+
+
+@pytest.mark.parametrize("e", [-50, -59, -62, -66])
+@pytest.mark.parametrize("m,k,n", [(256, 256, 256), (300, 512, 1024), (2048, 256, 2048)])
+def test_products_in_the_subnormal_range(lc, m, k, n, e):
+    """Operands near 2^e fit the planes, and their small products lie below 2^-126
+    from e = -55 on: they count in full (a sum below 2^-126 keeps steps of 2^-149),
+    where flushing them to zero would cost 2^-8 of the result."""
+    rng = np.random.default_rng(11)
+    scale = np.float32(2.0) ** np.float32(e)
+    a = rng.standard_normal((m, k), dtype=np.float32) * scale
+    b = rng.standard_normal((k, n), dtype=np.float32) * scale
+    s = lc.MatMulResidentSession(m, k, n)
+    s.start_into(a, b)
+    got = _exact64(s.finish_into()).reshape(m, n)
+    assert "split" in s.kernel_name()
+    s.close()
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    bound = (6 * k / 32 + 16) * 2.0 ** -23 * (np.abs(a) @ np.abs(b)) + (6 * k + 16) * 2.0 ** -149
+    assert (np.abs(got - a @ b) <= bound).all()

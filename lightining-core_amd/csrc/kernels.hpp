@@ -312,7 +312,7 @@ hipError_t gemmHalfTNHalfOut(const uint16_t* A, const uint16_t* Bt, uint16_t* C,
 hipError_t patchEmbedGemm(const uint16_t* x, const uint16_t* Wt, uint16_t* tokens, int B, int C, int H, int W, int P,
                           int E, Half t, hipStream_t stream);
 // The patch-embed conv as a row-major GEMM on vitPatchify's xp [M][K]:
-// tokens = relu(xp . Wt^T), the same tiles and k order as patchEmbedGemm.
+// tokens = relu(xp . Wt^T), the same k order as patchEmbedGemm.
 hipError_t patchTokensGemm(const uint16_t* xp, const uint16_t* Wt, uint16_t* tokens, int M, int K, int E, Half t,
                            int cus, hipStream_t stream);
 // QKV projection for the ViT block: qkv = tokens[M, E] . Wqkv_t[3E, E]^T with

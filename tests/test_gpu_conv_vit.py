@@ -175,9 +175,8 @@ def test_vit_block_small(lc, oracle, dtype):
     assert_parity(ref, got.reshape(ref.shape), dtype, f"vit small {dtype}")
 
 
-# Shapes for the ring-pipelined ViT GEMMs: P = 8 and 32 patch sources, token
-# counts that are not tile multiples (rows clamped), and T % 4 != 0, which
-# sends the QKV projection to the element-wise epilogue.
+# Shapes for the ViT GEMMs: P = 8 and 32 patch rows, token counts that are not
+# tile multiples (rows clamped), images that share a row block (T % 4 != 0).
 @pytest.mark.parametrize("bn,img,p,e,heads,dtype", [
     (3, 40, 8, 128, 2, "f16"),     # T = 25 (T % 4 != 0), M = 75
     (5, 96, 16, 192, 3, "bf16"),   # T = 36, M = 180, three heads of 64
@@ -194,8 +193,7 @@ def test_vit_block_shapes(lc, oracle, bn, img, p, e, heads, dtype):
 
 def test_vit_block_ring_off_matches(lc, monkeypatch):
     # CJ_HIP_VIT_RING=0 keeps the register-staged GEMMs: same inputs, results
-    # within the 16-bit tolerance of the ring path (the k order of the
-    # accumulation is the same; only the tiling differs).
+    # within the 16-bit tolerance of the ring tiles'.
     bn, c, img, p, e, heads = 2, 3, 64, 16, 128, 2
     x, w_conv, w_qkv, w_o = _vit_inputs(bn, c, img, p, e)
     ring = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype="f16")
@@ -206,65 +204,57 @@ def test_vit_block_ring_off_matches(lc, monkeypatch):
 
 @pytest.mark.parametrize("p,e", [(16, 128), (32, 256), (8, 128)])
 def test_vit_block_ring_stage_depth_bitwise(lc, monkeypatch, p, e):
-    # The patch and output GEMMs take 128-deep ring stages when K allows
-    # (CJ_HIP_VIT_RING_BK=64 forces 64): same k order, so the same bits.  P = 8
-    # keeps 64-deep stages for the patch GEMM (a 128-deep stage would span
-    # two channels) and checks that path too.
+    # The implicit-im2col patch GEMM (CJ_HIP_VIT_PATCHIFY=0) takes 128-deep ring
+    # stages when K allows (CJ_HIP_VIT_RING_BK=64 forces 64): same k order, so the
+    # same bits.  P = 8 keeps 64-deep stages either way (a 128-deep stage would
+    # span two channels).
     bn, c, img, heads = 2, 3, 64, 2
     x, w_conv, w_qkv, w_o = _vit_inputs(bn, c, img, p, e)
+    monkeypatch.setenv("CJ_HIP_VIT_PATCHIFY", "0")
     deep = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype="f16")
     monkeypatch.setenv("CJ_HIP_VIT_RING_BK", "64")
     shallow = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype="f16")
     np.testing.assert_array_equal(deep, shallow)
 
 
-# The fused QKV-projection + attention kernel (default where head dim is 64
-# and T <= 224) against the separate QKV GEMM and attention kernels
-# (CJ_HIP_VIT_FUSED=0): the projection accumulates in the same k order and the
-# attention runs the same per-wave arithmetic, so the bits match.  T = 25, 9
-# and 169 are not multiples of 4 or 64; T = 196 is config 4's.
-@pytest.mark.parametrize("bn,img,p,e,heads,dtype", [
-    (2, 64, 16, 128, 2, "f16"),    # T = 16
-    (3, 40, 8, 128, 2, "f16"),     # T = 25
-    (5, 96, 16, 192, 3, "bf16"),   # T = 36
-    (1, 48, 16, 128, 2, "bf16"),   # T = 9
-    (1, 208, 16, 128, 2, "f16"),   # T = 169
-    (2, 224, 16, 768, 12, "bf16"),  # config 4's image and width, T = 196
-])
-def test_vit_block_fused_matches_unfused(lc, monkeypatch, bn, img, p, e, heads, dtype):
-    note(f"[case] vit fused vs unfused bn={bn} img={img} p={p} e={e} heads={heads} {dtype}")
-    x, w_conv, w_qkv, w_o = _vit_inputs(bn, 3, img, p, e)
-    fused = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype=dtype)
-    monkeypatch.setenv("CJ_HIP_VIT_FUSED", "0")
-    unfused = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype=dtype)
-    np.testing.assert_array_equal(fused, unfused)
-
-
-# The fused kernel's edges: one 64-deep k-stage (E = 64, one head) and the
-# largest token count it takes (T = 224 = 14 x 16 patches of a 224 x 256
-# image: seven full query blocks, keys 224..255 padding), each bit-identical to
-# the separate kernels and, for T = 224, against the oracle on the whole block.
+# The QKV projection's head-major Q / K and transposed V stores and the attention
+# that reads them, against the oracle: token counts around a 4-, 16- and 64-row
+# boundary, one 64-wide head (E = 64), and the largest count with key padding in
+# the last tile (T = 224).
 @pytest.mark.parametrize("bn,ih,iw,p,e,heads,dtype", [
-    (2, 32, 32, 8, 64, 1, "f16"),     # T = 16, E = 64
+    (2, 64, 64, 16, 128, 2, "f16"),     # T = 16
+    (3, 40, 40, 8, 128, 2, "f16"),      # T = 25
+    (5, 96, 96, 16, 192, 3, "bf16"),    # T = 36
+    (1, 48, 48, 16, 128, 2, "bf16"),    # T = 9
+    (1, 208, 208, 16, 128, 2, "f16"),   # T = 169
+    (2, 32, 32, 8, 64, 1, "f16"),       # T = 16, E = 64
     (1, 224, 256, 16, 128, 2, "bf16"),  # T = 224
 ])
-def test_vit_block_fused_edges(lc, oracle, monkeypatch, bn, ih, iw, p, e, heads, dtype):
-    note(f"[case] vit fused edges bn={bn} {ih}x{iw} p={p} e={e} heads={heads} {dtype}")
+def test_vit_block_token_counts(lc, oracle, bn, ih, iw, p, e, heads, dtype):
+    note(f"[case] vit tokens bn={bn} {ih}x{iw} p={p} e={e} heads={heads} {dtype}")
     x = synth.uniform((bn, 3, ih, iw), lo=0.0, hi=1.0, stream=34)
     w_conv = synth.normal((e, 3, p, p), std=0.02, stream=35)
     w_qkv = synth.normal((e, 3 * e), std=0.02, stream=36)
     w_o = synth.normal((e, e), std=0.02, stream=37)
-    fused = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype=dtype)
+    got = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype=dtype)
     ref = oracle.vit_block(*(synth.round_to(t, dtype) for t in (x, w_conv, w_qkv, w_o)), heads)
-    assert_parity(ref, fused.reshape(ref.shape), dtype, f"vit fused {ih}x{iw} e{e} {dtype}")
-    monkeypatch.setenv("CJ_HIP_VIT_FUSED", "0")
-    unfused = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype=dtype)
-    np.testing.assert_array_equal(fused, unfused)
+    assert_parity(ref, got.reshape(ref.shape), dtype, f"vit tokens {ih}x{iw} e{e} {dtype}")
+
+
+# The benchmark's image and width (T = 196), first and last image, in bf16.
+def test_vit_block_bf16_two_images(lc, oracle):
+    bn, img, p, e, heads = 2, 224, 16, 768, 12
+    x, w_conv, w_qkv, w_o = _vit_inputs(bn, 3, img, p, e)
+    got = lc.vit_block(x, w_conv, w_qkv, w_o, heads, compute_dtype="bf16").reshape(bn * 196, e)
+    rounded = [synth.round_to(t, "bf16") for t in (x, w_conv, w_qkv, w_o)]
+    for i in range(bn):
+        rows = (i * 196, (i + 1) * 196)
+        assert_parity(oracle.vit_block(*rounded, heads, rows=rows), got[rows[0]:rows[1]], "bf16", f"vit image {i}")
 
 
 # The input stored as patch rows with the patch conv as a row-major GEMM (the
 # default) against the implicit-im2col GEMM on the NCHW image
-# (CJ_HIP_VIT_PATCHIFY=0): same tiles and k order, so the same bits.  Shapes:
+# (CJ_HIP_VIT_PATCHIFY=0): the same k order, so the same bits.  Shapes:
 # P = 8, 16 and 32, an image that is not a multiple of the patch (the last
 # 8 columns and rows are not covered), non-square.
 @pytest.mark.parametrize("bn,ih,iw,p,e,heads,dtype", [

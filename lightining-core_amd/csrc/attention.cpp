@@ -339,6 +339,12 @@ namespace {
 // small enough for the 16-query kernel (4 heads of S = 256: 7.5 against 12.6
 // us), nor one head up to S = 2048 at D <= 64, where that kernel and the
 // 32-query kernel's key splits are as fast (S = 2048: 23.2 against 23.4 us).
+// Everywhere else it beat that kernel and its key splits (200 shapes, 1 to 64
+// heads).  One head, S = 64 / 256 / 1024 / 4096, us: D = 96 15.2 /
+// 20.9 / 30.4 / 338 -> 8.6 / 15.2 / 23.9 / 57.9, D = 128 16.3 / 22.1 / 32.8 / 449
+// -> 10.7 / 17.2 / 27.3 / 69.0.  A call that uploads all of Q, K and V for one
+// launch, planes included, took no longer at any of 142 shapes (1x16x200x128
+// 224 -> 220 us, 1x1x2100x32 90 -> 90).
 // The planes take 4.5 times a tensor's fp32 bytes: at most an eighth of memory,
 // and they are given up when another allocation needs it.
 bool splitServes(const HipContext* ctx, const AttnShape& sh) {

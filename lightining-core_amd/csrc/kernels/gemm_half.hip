@@ -99,11 +99,11 @@ struct StoreQkv {
 // stage's fragments into registers during the stage before it, so a stage is
 // one barrier and its slot is free for the copies of the stage four ahead as
 // soon as the barrier is passed.
-// Bound: LDS bandwidth for the 128- and 96-row tiles (a stage reads and writes
-// 84-96 KB for 24-32 MFMAs a wave, 670-770 cycles at 128 bytes a cycle against
-// 384-512 of MFMA; measured 0.43-0.45 us a stage), the stream of Bt from HBM
-// for few rows.  The k order of every accumulator is that of the 256x256
-// kernels, so results agree bit for bit.
+// Bound: the copies and the barrier of each stage for the 128- and 96-row tiles
+// (24-32 MFMAs a wave, 384-512 cycles, in a stage of 0.43-0.45 us: one wave per
+// SIMD, MFMAs busy 50-55% of a CU's cycles and LDS reads 30%, no bank conflicts,
+// at 1500x3000x2000), the stream of Bt from HBM for few rows.  The k order of
+// every accumulator is that of the 256x256 kernels, so results agree bit for bit.
 // Measured against the best of the register-staged kernels and w4h, f16
 // (M x K x N, us): 1500x3000x2000 38.4 -> 24.4 (96x128); 2048^3 32.7 -> 23.5
 // (128x128); 1000x4096x4096 56.8 -> 38.6; 1024^3 8.6 -> 6.0 (64x64);

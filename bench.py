@@ -557,15 +557,17 @@ def bench_extras(lc, synth, cpu):
 # --pmc-workload`: the copy kernel behind a device-to-device lcMemcpy moves a
 # known number of bytes each way, which calibrates each counter; the GEMM's
 # per-dispatch means times those factors give its HBM traffic.  Figures from
-# profiles/gemm_f32_lds_kernel_1024cube_traffic.txt (update them when the kernel
+# profiles/gemm_f32_lds_kernel_1024cube_traffic.txt and
+# profiles/counters_fp32_planes_and_ring_tiles.txt (update them when a kernel
 # changes).
 PMC_COPY_BYTES = 256 << 20
 PMC_COPIES = 10
 PMC_GEMMS = 20
-# FETCH_SIZE: GEMM 12329.9 KiB/dispatch, copy 131084.4 KiB for 262144 KiB moved (x2.000);
-# WRITE_SIZE: GEMM 4096.0 KiB/dispatch, copy 262144.0 KiB (x1.000).
+# FETCH_SIZE: gemm_f32_lds_kernel 12323.0 KiB/dispatch, gemm_f32_split_kernel 18511.5, copy 131084.4 KiB for
+# 262144 KiB moved (x1.9998); WRITE_SIZE: 4096.0 KiB/dispatch, copy 262144.0 KiB (x1.000).
 # HBM bytes per launch (fetch + write, calibrated); other kernels report null.
-GEMM_F32_1024_TRAFFIC = {"gemm_f32_lds_kernel": 25235186 + 4194304}
+GEMM_F32_1024_TRAFFIC = {"gemm_f32_lds_kernel": 25235186 + 4194304,
+                         "gemm_f32_split_kernel": 37907959 + 4194304}
 # 8192^3 bf16, HBM bytes per launch (fetch + write, calibrated), per kernel:
 # profiles/gemm_half_tn_w4h_kernel_8192cube_traffic.txt: FETCH_SIZE 787628.8 KiB/dispatch (x1.9998),
 # WRITE_SIZE 262144.0 KiB (x1.000).  A kernel without its own counter passes (a variant forced by

@@ -112,8 +112,7 @@ __global__ __launch_bounds__(256) void attn_planes_kernel(const float* __restric
 // max over the four lanes that share a query.
 __device__ __forceinline__ float max_quads(float x) {
   const uint32_t u = __builtin_bit_cast(uint32_t, x);
-  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  return max_xor32(fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1])));
+  return max_xor32(max_of_swap(__builtin_amdgcn_permlane16_swap(u, u, false, false)));
 }
 
 // ---------------------------------------------------------------------------

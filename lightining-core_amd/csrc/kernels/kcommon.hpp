@@ -90,11 +90,19 @@ __device__ __forceinline__ float add_pair<F16>(uint32_t pair, float acc) {
   return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pair), ones, acc, false);
 }
 
+// The larger of a lane swap's two results.  They go through scalars first:
+// __builtin_bit_cast of a vector's element reads element 0 whatever the index.
+template <typename Pair>
+__device__ __forceinline__ float max_of_swap(Pair r) {
+  const uint32_t a = r[0];
+  const uint32_t b = r[1];
+  return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+
 // max over lanes l and l ^ 32 (v_permlane32_swap: no LDS round trip).
 __device__ __forceinline__ float max_xor32(float v) {
   const uint32_t u = __builtin_bit_cast(uint32_t, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+  return max_of_swap(__builtin_amdgcn_permlane32_swap(u, u, false, false));
 }
 
 // 32x32x16 MFMA on 8 packed 16-bit values per lane (as four dwords).

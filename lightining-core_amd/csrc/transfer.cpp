@@ -51,7 +51,7 @@ struct Transfer {
   std::size_t bytes = 0, chunk = 0;
   int n = 0;
   int threads = 1;             // that share the slots: thread w has slots w, w + threads, ...
-  int first = 0, end = 0;      // the chunks they move; first is a multiple of kSlots
+  int first = 0, end = 0;      // the chunks they move
   std::atomic<int> error{0};   // first hipError_t; everyone stops
 
   std::size_t size(int i) const { return i + 1 < n ? chunk : bytes - static_cast<std::size_t>(i) * chunk; }
@@ -92,18 +92,28 @@ class Engine {
       if (e != hipSuccess) {
         t.fail(e);
       }
-    } else if (hipStreamQuery(ctx->stream) != hipSuccess) {
-      // The stream is busy: the caller fills the ring alone, and the helpers are
-      // woken once its first slot is free again.
+    } else {
+      // While the stream is busy with earlier work the caller fills the ring
+      // alone, and the helpers are woken once the stream has come this far.  An
+      // event tells: after a hipStreamQuery that finds the stream busy, the copies
+      // that follow run at half the rate (2 x 256 MB 28.7 against 14.2 ms).
+      hipError_t e = hipEventRecord(reached_, ctx->stream);
+      bool busy = e == hipSuccess && hipEventQuery(reached_) == hipErrorNotReady;
+      t.end = 0;
+      while (busy && t.end < kSlots && t.end < t.n && !t.failed()) {
+        t.first = t.end++;
+        work(t, 0);
+        busy = hipEventQuery(reached_) == hipErrorNotReady;
+      }
       (void)hipGetLastError();
-      t.end = kSlots < t.n ? kSlots : t.n;
-      work(t, 0);
-      t.first = t.end;
-      t.end = t.n;
-      const hipError_t e = t.failed() ? hipSuccess : hipEventSynchronize(events_[0]);
+      if (busy) {
+        e = hipEventSynchronize(reached_);
+      }
       if (e != hipSuccess) {
         t.fail(e);
       }
+      t.first = t.end;
+      t.end = t.n;
     }
     if (t.failed()) {
       return static_cast<hipError_t>(t.error.load());
@@ -141,6 +151,9 @@ class Engine {
         return;
       }
     }
+    if (hipEventCreateWithFlags(&reached_, hipEventDisableTiming) != hipSuccess) {
+      return;
+    }
     // Helpers take no signals: those stay with the program's own threads.
     sigset_t all, before;
     sigfillset(&all);
@@ -173,27 +186,28 @@ class Engine {
   }
 
   void work(Transfer& t, int w) {
-    for (int first = t.first; first < t.end; first += kSlots) {
-      for (int s = w; s < kSlots && first + s < t.end; s += t.threads) {
-        const int i = first + s;
-        if (t.failed()) {
-          return;
+    for (int i = t.first; i < t.end; ++i) {
+      const int s = i % kSlots;
+      if (s % t.threads != w) {
+        continue;
+      }
+      if (t.failed()) {
+        return;
+      }
+      const hipError_t e = hipEventSynchronize(events_[s]);
+      if (e != hipSuccess) {
+        t.fail(e);
+        return;
+      }
+      char* host = t.host + static_cast<std::size_t>(i) * t.chunk;
+      if (t.down) {
+        std::memcpy(host, slot(i), t.size(i));
+        if (i + kSlots < t.n) {
+          enqueue(t, i + kSlots);
         }
-        const hipError_t e = hipEventSynchronize(events_[s]);
-        if (e != hipSuccess) {
-          t.fail(e);
-          return;
-        }
-        char* host = t.host + static_cast<std::size_t>(i) * t.chunk;
-        if (t.down) {
-          std::memcpy(host, slot(i), t.size(i));
-          if (i + kSlots < t.n) {
-            enqueue(t, i + kSlots);
-          }
-        } else {
-          std::memcpy(slot(i), host, t.size(i));
-          enqueue(t, i);
-        }
+      } else {
+        std::memcpy(slot(i), host, t.size(i));
+        enqueue(t, i);
       }
     }
   }
@@ -220,6 +234,7 @@ class Engine {
 
   PinnedBuffer ring_;
   hipEvent_t events_[kSlots] = {};
+  hipEvent_t reached_ = nullptr;  // recorded before an upload
   int helpers_ = 0;
   const pid_t pid_ = getpid();
   std::mutex run_mu_;  // one copy at a time

@@ -95,6 +95,26 @@ def test_upload_behind_queued_work(lc):
     busy.close()
 
 
+def test_upload_to_new_buffers_keeps_its_rate(lc):
+    """A new session's first kernels make its stream busy for a moment before its
+    operands go up: they take as long as into the session's buffers later (the
+    allocations and fills between them are 3% of it; half the rate would be twice)."""
+    n = 8192
+    a = np.ones((n, n), np.float32)
+    fresh, again = [], []
+    for _ in range(6):
+        s = lc.MatMulResidentSession(n, n, n, "bf16")
+        for times in (fresh, again):
+            begin = time.perf_counter()
+            s.start_into(a, a)
+            times.append(time.perf_counter() - begin)
+            s.sync_into()
+        s.close()
+    fresh, again = (sorted(times[1:])[2] for times in (fresh, again))  # the first call also times variants
+    note(f"[transfer] 2 x 256 MB into new buffers {fresh * 1e3:.1f} ms, again {again * 1e3:.1f} ms")
+    assert fresh < 1.6 * again
+
+
 def test_pinned_result_buffer(lc):
     hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime the backend has loaded
     rows = 2 * MIB + 5
